@@ -13,6 +13,7 @@
 
 #include "mbvh_common.h"
 #include "mbvh_kernels.h"
+#include "mbvh_frame.h"
 
 using namespace mbvh;
 
@@ -125,6 +126,7 @@ struct mbvh_mesh {
   uint2* d_root_slots = nullptr;    // slot range (first, end) of each root
   uint2* d_bigleaf = nullptr;
   float4* d_tris = nullptr;
+  float4* d_frames = nullptr;       // kFrameRows per slot, written from d_tris on the device
   uint32_t* d_vidx = nullptr;
   uint32_t* d_face_slot = nullptr;  // indirect meshes: face -> slot (0xFFFFFFFF if absent)
   float4* d_nodes4 = nullptr;       // 4-wide tree
@@ -427,6 +429,7 @@ void free_mesh_buffers(mbvh_mesh* m) {
   if (m->d_root_slots) (void)hipFree(m->d_root_slots);
   if (m->d_bigleaf) (void)hipFree(m->d_bigleaf);
   if (m->d_tris) (void)hipFree(m->d_tris);
+  if (m->d_frames) (void)hipFree(m->d_frames);
   if (m->d_vidx) (void)hipFree(m->d_vidx);
   if (m->d_face_slot) (void)hipFree(m->d_face_slot);
   if (m->d_nodes4) (void)hipFree(m->d_nodes4);
@@ -451,6 +454,7 @@ void free_mesh_buffers(mbvh_mesh* m) {
   m->d_roots = nullptr;
   m->d_bigleaf = nullptr;
   m->d_tris = nullptr;
+  m->d_frames = nullptr;
   m->d_vidx = nullptr;
 }
 
@@ -464,6 +468,7 @@ MeshView view_of(const mbvh_mesh* m) {
   v.max_stack4 = m->max_stack4;
   v.bigleaf = m->d_bigleaf;
   v.tris = m->d_tris;
+  v.frames = m->d_frames;
   v.n_roots = m->n_roots;
   v.max_stack = m->max_stack;
   v.coord_max = m->d_coord_max;
@@ -799,6 +804,12 @@ extern "C" int mbvh_mesh_upload(mbvh_ctx* ctx, const void* const* roots, const u
     for (uint64_t sl = 0; sl < n_slots; sl++) face_slot[tris_face(tris, sl)] = static_cast<uint32_t>(sl);
     rc = upload(reinterpret_cast<void**>(&m->d_face_slot), face_slot.data(), face_slot.size() * sizeof(uint32_t));
   }
+  if (!rc) rc = upload(reinterpret_cast<void**>(&m->d_frames), nullptr, kFrameRows * n_slots * sizeof(float4));
+  if (!rc) {
+    hipError_t e = launch_tri_frames(m->d_tris, n_slots, m->d_frames, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) rc = set_error(MBVH_ERR_HIP, "mbvh_mesh_upload: triangle frames failed (%s)", hipGetErrorString(e));
+  }
   if (rc) {
     free_mesh_buffers(m);
     m->magic = 0;
@@ -893,6 +904,7 @@ int enqueue_refit(mbvh_mesh* mesh, const float* d_positions, uint64_t vertex_cou
   a.four_map = mesh->d_four_map;
   a.n_four = mesh->n_four_map;
   a.tris = mesh->d_tris;
+  a.frames = mesh->d_frames;
   a.vidx = mesh->d_vidx;
   a.n_slots = mesh->n_slots;
   a.positions = d_positions;

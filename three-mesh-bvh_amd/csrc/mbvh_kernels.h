@@ -17,6 +17,7 @@ struct MeshView {
   uint32_t max_stack4;    // stack entries a quad traversal can need (4-wide or binary)
   const uint2* bigleaf;
   const float4* tris;  // 3 per slot
+  const float4* frames;  // kFrameRows per slot: each triangle in its own plane (closest point)
   uint32_t n_roots;
   uint32_t max_stack;  // stack entries a traversal of this mesh can need
   const float* coord_max;  // device: an upper bound of |vertex coordinate| (scales FP32 error bounds;
@@ -124,6 +125,7 @@ struct RefitArgs {
   const uint2* four_map;      // (float offset in the 4-wide tree, float offset in the wide nodes)
   uint64_t n_four;
   float4* tris;
+  float4* frames;             // rewritten with the triangles
   const uint32_t* vidx;
   uint64_t n_slots;
   const float* positions;     // new vertex positions (device)
@@ -139,6 +141,8 @@ struct RefitArgs {
   uint32_t n_roots;
 };
 hipError_t launch_refit(const RefitArgs& a, hipStream_t s);
+// The frames of uploaded triangles (kFrameRows float4 per slot).
+hipError_t launch_tri_frames(const float4* tris, uint64_t n_slots, float4* frames, hipStream_t s);
 
 // ---- device build -------------------------------------------------------------------------------
 // Positions q in [0, span) of the primitive buffer being built; a non-indirect build's buffer is the

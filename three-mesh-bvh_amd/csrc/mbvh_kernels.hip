@@ -15,6 +15,7 @@
 // equal minima, which is the reference's strict-< rule.
 #include "mbvh_kernels.h"
 #include "mbvh_closest_ff.h"
+#include "mbvh_frame.h"
 
 namespace mbvh {
 namespace {
@@ -416,14 +417,22 @@ struct Cands {
   __device__ __forceinline__ uint2 get(int i) const { return sh_cand[i * kBlock + lane]; }
   // Drops candidates with lb > U, keeping order. Returns true if a slot is free afterwards.
   __device__ __forceinline__ bool compact(float U) {
+    int at = 0;
+    return compact(U, at);
+  }
+  // The same; `at`, a position in the list, stays between the same entries.
+  __device__ __forceinline__ bool compact(float U, int& at) {
     int m = 0;
+    const int before = at;
     for (int i = 0; i < n; i++) {
+      if (i == before) at = m;
       const uint2 e = get(i);
       if (__uint_as_float(e.y) <= U || !(__uint_as_float(e.y) == __uint_as_float(e.y))) {
         if (m != i) put(m, e.x, __uint_as_float(e.y));
         m++;
       }
     }
+    if (before >= n) at = m;
     n = m;
     return n < kCand;
   }
@@ -1553,6 +1562,22 @@ __device__ __forceinline__ float query_error(f3 q, f3 ql, float coord_max) {
   return e;
 }
 
+// For a double query, twice its distance to q: bounds measured from q widened by it also bound the
+// distances from q + ql, and the boxes pruned from q stay pruned.
+__device__ __forceinline__ float query_shift(f3 ql) {
+  return 2.0f * (fabsf(ql.x) + fabsf(ql.y) + fabsf(ql.z)) * (1.0f + 4.0f * kU);
+}
+
+// The error bound of a frame's FP32 squared distance d2 (w: the frame's f0.w); with a query shift e
+// it grows by 2 d e + 2 e^2 (the cross term of e and the frame's own error is inside that square).
+template <bool kLo>
+__device__ __forceinline__ float frame_error(float d2, float w, float e) {
+  float e2 = fmaf(kFrameRel, d2, fabsf(w));
+  if (kLo) e2 += (2.0f * sqrt_up(d2) + 2.0f * e) * e;
+  return e2;
+}
+__device__ __forceinline__ bool signbit_of(float w) { return __float_as_int(w) < 0; }
+
 // Whether a box (FP32 squared distance s from q) is entered under maxThreshold^2 (t2): the FP32
 // value decides when it is clear of its error band, double-float otherwise. Double queries always
 // decide in double-float (their FP32 score is measured from q, not from q + ql).
@@ -1598,7 +1623,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_closest_point4(ClosestPointArgs A
     if (qi >= A.n) continue;
     const f3 q = mk(A.points[3 * qi + 0], A.points[3 * qi + 1], A.points[3 * qi + 2]);
     const f3 ql = kLo ? load3(A.points_lo, qi) : mk(0.0f, 0.0f, 0.0f);
-    const float e_abs = query_error<kLo>(q, ql, *M.coord_max);
+    const float e_lo = kLo ? query_shift(ql) : 0.0f;
     float U = kInf;  // quad-wide upper bound of the best squared distance (after each leaf)
     bool overflow = false;
     Cands cl;
@@ -1633,25 +1658,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_closest_point4(ClosestPointArgs A
           leaf_range(ref, M.bigleaf, off, cnt);
           float Ul = U;
           for (uint32_t s = off + q4; s < off + cnt; s += 4) {
-            const Tri tr = load_tri(M.tris, s);
-            // the triangle's own box first: its squared distance (clamp exact, three roundings per
-            // axis and two in the sum, covered by 8 ulps) bounds the triangle's from below, so a
-            // box beyond the upper bound Ul rules the triangle out without the full test
-            const float sb = box_score(q, fminf(fminf(tr.p0.x, tr.p1.x), tr.p2.x), fminf(fminf(tr.p0.y, tr.p1.y), tr.p2.y),
-                                       fminf(fminf(tr.p0.z, tr.p1.z), tr.p2.z), fmaxf(fmaxf(tr.p0.x, tr.p1.x), tr.p2.x),
-                                       fmaxf(fmaxf(tr.p0.y, tr.p1.y), tr.p2.y), fmaxf(fmaxf(tr.p0.z, tr.p1.z), tr.p2.z));
-            if (sb * (1.0f - 8.0f * kU) > Ul) continue;
-            const f3 cp = closest_on_triangle(q, tr.a(), tr.b(), tr.c());
-            const f3 dv = sub(q, cp);
-            const float d2 = dot(dv, dv);
-            float lb = -kInf;  // FP32 failed (degenerate triangle, NaN): decide exactly at the end
-            if (d2 == d2) {
-              const float e2 = (2.0f * sqrt_up(d2) + e_abs) * e_abs + 4.0f * kU * d2;
-              lb = d2 - e2;
-              if (lb > Ul) continue;
-              // every candidate that may tie stays listed: ties go to the reference's first
-              Ul = fminf(Ul, d2 + e2);
-            }
+            const float4* const fr = M.frames + static_cast<uint64_t>(kFrameRows) * s;
+            const float4 f0 = fr[0];
+            const float d2 = frame_dist2(q, f0, fr[1], fr[2], fr[3], fr[4]);
+            const float e2 = frame_error<kLo>(d2, f0.w, e_lo);
+            const float lb = d2 - e2;  // NaN: the triangle is left to the exact step
+            if (lb > Ul) continue;
+            // every candidate that may tie stays listed: ties go to the reference's first
+            if (!signbit_of(f0.w)) Ul = fminf(Ul, d2 + e2);
             if (cl.n == kCand && !cl.compact(Ul)) {
               const Winner r = resolve_point<kLo, true>(cl, Ul, q, ql, M.tris, T);
               const uint32_t w = r.w;
@@ -1723,13 +1737,19 @@ __global__ __launch_bounds__(kBlock, 4) void k_closest_point4(ClosestPointArgs A
 // Closest point for coherent queries (grid samples, Morton-ordered point sets): a packet of 64
 // queries, one per lane of a wave, walks the 4-wide tree together. A child is entered when any
 // lane's query may need it (its squared box distance under that lane's upper bound and under
-// maxThreshold^2); node records and triangles are read at wave-uniform addresses (scalar loads),
+// maxThreshold^2); node records and triangle frames are read at wave-uniform addresses (scalar loads),
 // so the node and leaf steps run with every lane busy instead of one quad in three. Each lane keeps
-// its own bound and candidate list and resolves them exactly as the quad kernel does, so the
-// results are bit for bit those of k_closest_point4: the packet's order only steers the search.
-// Children are ordered by the scores of one lane near the middle of the packet. The stack (the
-// children's own 32-byte records, re-scored per lane on pop) lives in LDS; the host uses this
-// kernel only for trees whose 4-wide stack fits it.
+// its own bound and candidate list; k_closest_point_resolve settles the lists exactly as the quad
+// kernel does, so the results are bit for bit those of k_closest_point4: the packet's order only
+// steers the search. Children are ordered by the scores of one lane near the middle of the packet. The
+// stack lives in LDS; the host uses this kernel only for trees whose 4-wide stack fits it.
+//
+// What bounds it: issue, vector and scalar alike (a million-triangle sphere and a 256^3 grid: 1,354
+// triangles, 208 nodes and 240 pops per packet). Hence the triangle frames (44 vector instructions
+// and no branch per triangle; the tests for the seven regions of a triangle, each branch entered
+// by some lane, behind a box test took about 26 + 145), one held candidate instead of a list push and compaction per
+// improvement, children sorted by scalar selects, and popped children expanded without a second score:
+// 65.7 -> 43 ms for that grid's packets, 7.6 -> 5.2 ms for a 128^3 grid over 320,000 triangles.
 // ------------------------------------------------------------------------------------------
 constexpr int kPacketStack = static_cast<int>(kPacketStackEntries);
 constexpr uint32_t kPacketRedoMark = 0xFFFFFFFFu;   // cand_meta: the query went to the redo list
@@ -1743,16 +1763,29 @@ __device__ __forceinline__ float4 pick4(uint32_t k, float4 a, float4 b, float4 c
 typedef __attribute__((address_space(4))) const float ConstF;  // read-only for the launch: scalar loads
 __device__ __forceinline__ float4 cload4(ConstF* p) { return make_float4(p[0], p[1], p[2], p[3]); }
 
-template <bool kLo>
+// A packet's stack entry: the child's reference, and with a finite maxThreshold its box as well (the
+// leaf step then needs it per lane).
+template <bool kMax>
+struct PacketStack {
+  using Entry = uint32_t;
+};
+template <>
+struct PacketStack<true> {
+  struct Entry {
+    float4 r0, r1;
+  };
+};
+
+template <bool kLo, bool kMax>
 __global__ __launch_bounds__(kBlock, 8) void k_closest_point_packet(ClosestPointArgs A) {
-  __shared__ float4 pstack[(kBlock / 64) * kPacketStack * 2];
+  using Entry = typename PacketStack<kMax>::Entry;
+  __shared__ Entry pstack[(kBlock / 64) * kPacketStack];
   const uint32_t lane = threadIdx.x, wl = lane & 63u;
-  float4* const stk = pstack + (lane >> 6) * kPacketStack * 2;
+  Entry* const stk = pstack + (lane >> 6) * kPacketStack;
   const MeshView M = A.mesh;
   ConstF* const nodes4 = (ConstF*)(M.nodes4);
-  ConstF* const tris = (ConstF*)(M.tris);
-  const bool max_finite = A.max_threshold < kInf;
-  const ff max_t2 = max_finite ? thr_sq(A.max_threshold, A.max_lo) : ff{kInf, 0.0f};
+  ConstF* const frames = (ConstF*)(M.frames);
+  const ff max_t2 = kMax ? thr_sq(A.max_threshold, A.max_lo) : ff{kInf, 0.0f};
   constexpr float kScoreSlack = 1.0f - 4.0f * kU;
   const float qnan = __int_as_float(0x7fc00000);
 
@@ -1770,23 +1803,57 @@ __global__ __launch_bounds__(kBlock, 8) void k_closest_point_packet(ClosestPoint
       q = mk(A.points[3 * qi + 0], A.points[3 * qi + 1], A.points[3 * qi + 2]);
       if (kLo) ql = load3(A.points_lo, qi);
     }
-    const float e_abs = query_error<kLo>(q, ql, *M.coord_max);
-    float U = active ? kInf : -1.0f;  // this lane's upper bound of its best squared distance
+    const float e_lo = kLo ? query_shift(ql) : 0.0f;
+    float U = active ? kInf : -kInf;  // this lane's upper bound of its best squared distance
     const uint64_t act = __ballot(active);
     if (act == 0) continue;
     // the lane whose scores order the children: lane 32 if its query is live, else the first live one
     const uint32_t leader = (act >> 32) & 1u ? 32u : static_cast<uint32_t>(__builtin_ctzll(act));
-    // this query's candidates: a kCand-entry list in LDS, compacted against the bound when full; a
-    // candidate that finds it full of live ones goes onto the query's chain in the global pool
+    // this query's candidates, in visit order: the last triangle certainly nearer than the one held
+    // before it (its slot, lower bound and place among the others); and those that may tie with it, in
+    // a list in LDS, compacted against the bound when full; a candidate that finds it full of live
+    // ones goes onto the query's chain in the global pool
+    int near_at = 0;
+    uint32_t near_slot = kNoHit;
+    float near_lb = kInf;
     Cands cl;
     cl.lane = lane;
     cl.n = 0;
     uint32_t head = kPoolEnd;
     bool redo = false, overflow = false;
+
+    auto test = [&](uint32_t s, float4 f0, float4 f1, float4 f2, float4 f3, float4 f4, bool reach) __attribute__((always_inline)) {
+      const float d2 = frame_dist2(q, f0, f1, f2, f3, f4);
+      const float e2 = frame_error<kLo>(d2, f0.w, e_lo);
+      const float lb = d2 - e2;  // NaN: the triangle is left to the exact step
+      if (reach && !(lb > U)) {
+        const bool sure = !signbit_of(f0.w);
+        const float ub = d2 + e2;
+        if (sure) U = fminf(U, ub);
+        if (sure && ub < near_lb) {  // the one before can neither win nor tie
+          near_slot = s;
+          near_lb = lb;
+          if (cl.n) cl.compact(U);
+          near_at = cl.n;
+        } else if (cl.n < kCand - 1 || (cl.compact(U, near_at), cl.n < kCand - 1)) {  // one entry is the last triangle's
+          cl.put(cl.n++, s, lb);
+        } else {
+          const uint32_t at = atomicAdd(A.pool_count, 1u);
+          if (at < A.pool_cap) {
+            A.pool[at] = make_uint4(s, __float_as_uint(lb), head, 0u);
+            head = at;
+          } else {
+            redo = true;  // the pool ran out: the quad kernel finishes this query
+            U = -kInf;
+          }
+        }
+      }
+    };
+
     for (uint32_t r = 0; r < M.n_roots && !overflow; r++) {
       uint32_t ref = __builtin_amdgcn_readfirstlane(M.roots4[r]);
       int sp = 0;
-      // the current node's own box record (a root has none: roots are never bounds-tested)
+      // kMax: the current node's own box record (a root has none: roots are never bounds-tested)
       float4 cb0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), cb1 = cb0;
       bool has_box = false;
       while (ref != kDone) {
@@ -1796,47 +1863,54 @@ __global__ __launch_bounds__(kBlock, 8) void k_closest_point_packet(ClosestPoint
           // one per child), and the maxThreshold decisions, which may call out of line, come after
           ref = __builtin_amdgcn_readfirstlane(ref);
           ConstF* const nd = nodes4 + 32ull * ref;
-          uint32_t keys[4];
-          uint64_t need_any = 0;
           float4 rec0[4], rec1[4];
 #pragma unroll
           for (int k = 0; k < 4; k++) {
             rec0[k] = cload4(nd + 8 * k);
             rec1[k] = cload4(nd + 8 * k + 4);
           }
+          const float reachable = U * (1.0f + 8.0f * kU);  // the scores' roundings (4 ulps) taken to the bound
           float raw[4];
-          bool in[4];
+          uint64_t need[4];  // the lanes that enter each child
 #pragma unroll
           for (int k = 0; k < 4; k++) {
-            const uint32_t cref = __float_as_uint(rec1[k].z);
             raw[k] = box_score(q, rec0[k].x, rec0[k].y, rec0[k].z, rec0[k].w, rec1[k].x, rec1[k].y);
-            in[k] = cref != kDone && raw[k] * kScoreSlack <= U;
+            need[k] = __float_as_uint(rec1[k].z) != kDone ? __ballot(raw[k] <= reachable) : 0ull;
           }
-          if (max_finite) {
+          if (kMax) {
 #pragma unroll
-            for (int k = 0; k < 4; k++)
-              if (in[k])
-                in[k] = below_max<kLo>(true, raw[k], max_t2, q, ql, rec0[k].x, rec0[k].y, rec0[k].z, rec0[k].w,
-                                       rec1[k].x, rec1[k].y);
+            for (int k = 0; k < 4; k++) {
+              bool in = (need[k] >> wl) & 1u;
+              if (in) in = below_max<kLo>(true, raw[k], max_t2, q, ql, rec0[k].x, rec0[k].y, rec0[k].z, rec0[k].w,
+                                          rec1[k].x, rec1[k].y);
+              need[k] = __ballot(in);
+            }
           }
+          int nh = 0;
+          uint32_t keys[4], refs[4];
 #pragma unroll
           for (int k = 0; k < 4; k++) {
-            const uint64_t m = __ballot(in[k]);
-            need_any |= m ? (1ull << k) : 0ull;
+            nh += need[k] ? 1 : 0;
             // the leader's score (bits of a non-negative float order as unsigned) with the child's index
             const uint32_t kb = __builtin_amdgcn_readlane(__float_as_uint(raw[k]), leader);
-            keys[k] = m ? ((kb & ~3u) | static_cast<uint32_t>(k)) : 0xFFFFFFFFu;
+            keys[k] = need[k] ? ((kb & ~3u) | static_cast<uint32_t>(k)) : 0xFFFFFFFFu;
+            refs[k] = __float_as_uint(rec1[k].z);
           }
           // sort the (at most four) entered children nearest first
-#define MBVH_CSWAP(i, j)                  \
-  {                                       \
-    const uint32_t lo_ = min(keys[i], keys[j]); \
-    keys[j] = max(keys[i], keys[j]);      \
-    keys[i] = lo_;                        \
-  }
-          MBVH_CSWAP(0, 1) MBVH_CSWAP(2, 3) MBVH_CSWAP(0, 2) MBVH_CSWAP(1, 3) MBVH_CSWAP(1, 2)
-#undef MBVH_CSWAP
-          const int nh = __builtin_popcount(static_cast<uint32_t>(need_any));
+          auto cswap = [&](int i, int j) __attribute__((always_inline)) {
+            const bool x = keys[j] < keys[i];
+            const uint32_t ka = x ? keys[j] : keys[i], kb = x ? keys[i] : keys[j];
+            const uint32_t ra = x ? refs[j] : refs[i], rb = x ? refs[i] : refs[j];
+            keys[i] = ka;
+            keys[j] = kb;
+            refs[i] = ra;
+            refs[j] = rb;
+          };
+          cswap(0, 1);
+          cswap(2, 3);
+          cswap(0, 2);
+          cswap(1, 3);
+          cswap(1, 2);
           if (nh == 0) {
             ref = kDone;
           } else {
@@ -1845,18 +1919,27 @@ __global__ __launch_bounds__(kBlock, 8) void k_closest_point_packet(ClosestPoint
               break;
             }
             // push the farther entered children (farthest deepest), continue with the nearest
-            for (int i = nh - 1; i >= 1; i--) {
-              const uint32_t k = keys[i] & 3u;
-              if (wl == 0) {
-                stk[2 * sp] = pick4(k, rec0[0], rec0[1], rec0[2], rec0[3]);
-                stk[2 * sp + 1] = pick4(k, rec1[0], rec1[1], rec1[2], rec1[3]);
+#pragma unroll
+            for (int i = 3; i >= 1; i--) {
+              if (i >= nh) continue;
+              if constexpr (kMax) {
+                const uint32_t k = keys[i] & 3u;
+                if (wl == 0) {
+                  stk[sp].r0 = pick4(k, rec0[0], rec0[1], rec0[2], rec0[3]);
+                  stk[sp].r1 = pick4(k, rec1[0], rec1[1], rec1[2], rec1[3]);
+                }
+              } else {
+                if (wl == 0) stk[sp] = refs[i];
               }
               sp++;
             }
-            cb0 = pick4(keys[0] & 3u, rec0[0], rec0[1], rec0[2], rec0[3]);
-            cb1 = pick4(keys[0] & 3u, rec1[0], rec1[1], rec1[2], rec1[3]);
-            has_box = true;
-            ref = __float_as_uint(cb1.z);
+            if (kMax) {
+              const uint32_t k0 = keys[0] & 3u;
+              cb0 = pick4(k0, rec0[0], rec0[1], rec0[2], rec0[3]);
+              cb1 = pick4(k0, rec1[0], rec1[1], rec1[2], rec1[3]);
+              has_box = true;
+            }
+            ref = refs[0];
           }
         } else {
           // ---- leaf step: every lane tests its query against each triangle ----
@@ -1865,85 +1948,57 @@ __global__ __launch_bounds__(kBlock, 8) void k_closest_point_packet(ClosestPoint
           // the packet entered this leaf for some lane; a lane whose maxThreshold excludes the leaf's
           // box (and so, the boxes nesting, the leaf) must not record its triangles
           bool reach = active;
-          if (reach && max_finite && has_box) {
+          if (kMax && reach && has_box) {
             const float raw = box_score(q, cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y);
             reach = below_max<kLo>(true, raw, max_t2, q, ql, cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y);
           }
-          // the leaf (and so its range) is the packet's: the walk stays in scalar registers, and the
-          // next triangle's scalar loads are issued before this one is tested so that their latency
-          // overlaps the test instead of stalling the wave at the top of every iteration
+          // the leaf (and so its range) is the packet's: the walk stays in scalar registers. Two
+          // triangles' rows are loaded at a time; the other waves cover the loads (rotating a
+          // prefetched triangle through scalar registers costs 20 moves each, as much as it hides)
           off = __builtin_amdgcn_readfirstlane(off);
           cnt = __builtin_amdgcn_readfirstlane(cnt);
-          ConstF* tp = tris + 12ull * off;
-          Tri nx;
-          if (cnt) {
-            nx.p0 = cload4(tp);
-            nx.p1 = cload4(tp + 4);
-            nx.p2 = cload4(tp + 8);
-          }
-          for (uint32_t k = 0; k < cnt; k++) {
-            const uint32_t s = off + k;
-            const Tri tr = nx;
-            tp += 12;
-            if (k + 1 < cnt) {
-              nx.p0 = cload4(tp);
-              nx.p1 = cload4(tp + 4);
-              nx.p2 = cload4(tp + 8);
-            }
-            const float sb = box_score(q, fminf(fminf(tr.p0.x, tr.p1.x), tr.p2.x), fminf(fminf(tr.p0.y, tr.p1.y), tr.p2.y),
-                                       fminf(fminf(tr.p0.z, tr.p1.z), tr.p2.z), fmaxf(fmaxf(tr.p0.x, tr.p1.x), tr.p2.x),
-                                       fmaxf(fmaxf(tr.p0.y, tr.p1.y), tr.p2.y), fmaxf(fmaxf(tr.p0.z, tr.p1.z), tr.p2.z));
-            const bool near = reach && sb * (1.0f - 8.0f * kU) <= U;
-            if (__ballot(near) == 0) continue;
-            if (near) {
-              const f3 cp = closest_on_triangle(q, tr.a(), tr.b(), tr.c());
-              const f3 dv = sub(q, cp);
-              const float d2 = dot(dv, dv);
-              float lb = -kInf;  // FP32 failed (degenerate triangle, NaN): decide exactly at the end
-              bool add = true;
-              if (d2 == d2) {
-                const float e2 = (2.0f * sqrt_up(d2) + e_abs) * e_abs + 4.0f * kU * d2;
-                lb = d2 - e2;
-                add = lb <= U;
-                if (add) U = fminf(U, d2 + e2);
-              }
-              if (add) {
-                if (cl.n < kCand || cl.compact(U)) {
-                  cl.put(cl.n++, s, lb);
-                } else {
-                  const uint32_t at = atomicAdd(A.pool_count, 1u);
-                  if (at < A.pool_cap) {
-                    A.pool[at] = make_uint4(s, __float_as_uint(lb), head, 0u);
-                    head = at;
-                  } else {
-                    redo = true;  // the pool ran out: the quad kernel finishes this query
-                    U = -1.0f;
-                  }
-                }
-              }
-            }
+          for (uint32_t k = 0; k < cnt; k += 2) {
+            ConstF* const tp = frames + 4ull * kFrameRows * (off + k);
+            const bool two = k + 1 < cnt;
+            ConstF* const tq = two ? tp + 4 * kFrameRows : tp;
+            float4 fa[kFrameRows], fb[kFrameRows];
+#pragma unroll
+            for (int r = 0; r < kFrameRows; r++) fa[r] = cload4(tp + 4 * r);
+#pragma unroll
+            for (int r = 0; r < kFrameRows; r++) fb[r] = cload4(tq + 4 * r);
+            test(off + k, fa[0], fa[1], fa[2], fa[3], fa[4], reach);
+            if (two) test(off + k + 1, fb[0], fb[1], fb[2], fb[3], fb[4], reach);
           }
           ref = kDone;
         }
-        // ---- pop: the nearest pushed child some lane still needs ----
+        // ---- pop: the nearest pushed child; with maxThreshold, the nearest some lane still needs (a
+        // child no lane needs any more is rare, 10 of 240 pops on the million-triangle grid: expanding
+        // it costs less than scoring every popped box again) ----
         while (ref == kDone && sp > 0) {
           sp--;
-          const float4 e0 = stk[2 * sp], e1 = stk[2 * sp + 1];
-          const float raw = box_score(q, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y);
-          bool in = raw * kScoreSlack <= U;
-          if (in && max_finite) in = below_max<kLo>(true, raw, max_t2, q, ql, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y);
-          if (__ballot(in)) {
-            cb0 = e0;
-            cb1 = e1;
-            has_box = true;
-            ref = __builtin_amdgcn_readfirstlane(__float_as_uint(e1.z));
+          if constexpr (kMax) {
+            const float4 e0 = stk[sp].r0, e1 = stk[sp].r1;
+            const float raw = box_score(q, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y);
+            bool in = raw * kScoreSlack <= U;
+            if (in) in = below_max<kLo>(true, raw, max_t2, q, ql, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y);
+            if (__ballot(in)) {
+              cb0 = e0;
+              cb1 = e1;
+              has_box = true;
+              ref = __builtin_amdgcn_readfirstlane(__float_as_uint(e1.z));
+            }
+          } else {
+            ref = __builtin_amdgcn_readfirstlane(stk[sp]);
           }
         }
       }
     }
     if (active) {
       const uint64_t v = visit - A.tile0 * 64;
-      for (int c = 0; c < cl.n; c++) A.cand[v * kPacketCand + c] = cl.get(c);
+      const int held = near_slot != kNoHit ? 1 : 0;
+      if (held) A.cand[v * kPacketCand + near_at] = make_uint2(near_slot, __float_as_uint(near_lb));
+      for (int c = 0; c < cl.n; c++) A.cand[v * kPacketCand + c + (held && c >= near_at ? 1 : 0)] = cl.get(c);
+      cl.n += held;
       A.cand_meta[v] = make_uint4(overflow ? kPacketStackMark : (redo ? kPacketRedoMark : static_cast<uint32_t>(cl.n)),
                                   __float_as_uint(U), head, 0u);
       if (redo) A.redo[atomicAdd(A.redo_count, 1u)] = static_cast<uint32_t>(qi);
@@ -3822,13 +3877,19 @@ hipError_t launch_closest_point_packet(const ClosestPointArgs& a, uint64_t threa
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, a.pool_count);
   const dim3 grid(static_cast<uint32_t>(threads / kBlock));
   const dim3 rgrid(static_cast<uint32_t>((a.tiles * 64 + kBlock - 1) / kBlock));
-  if (a.points_lo) {
-    hipLaunchKernelGGL(k_closest_point_packet<true>, grid, dim3(kBlock), 0, s, a);
+  const bool lo = a.points_lo != nullptr, max = a.max_threshold < kInf;
+  if (lo && max)
+    hipLaunchKernelGGL((k_closest_point_packet<true, true>), grid, dim3(kBlock), 0, s, a);
+  else if (lo)
+    hipLaunchKernelGGL((k_closest_point_packet<true, false>), grid, dim3(kBlock), 0, s, a);
+  else if (max)
+    hipLaunchKernelGGL((k_closest_point_packet<false, true>), grid, dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_closest_point_packet<false, false>), grid, dim3(kBlock), 0, s, a);
+  if (lo)
     hipLaunchKernelGGL(k_closest_point_resolve<true>, rgrid, dim3(kBlock), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(k_closest_point_packet<false>, grid, dim3(kBlock), 0, s, a);
+  else
     hipLaunchKernelGGL(k_closest_point_resolve<false>, rgrid, dim3(kBlock), 0, s, a);
-  }
   return hipGetLastError();
 }
 

@@ -24,6 +24,7 @@
 // them by the changed flag; a node not visited keeps its box and counts as unchanged. The triangle
 // corners and the coordinate bound are refreshed everywhere, as the queries read the new positions.
 #include "mbvh_kernels.h"
+#include "mbvh_frame.h"
 
 namespace mbvh {
 namespace {
@@ -67,16 +68,29 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_bound(RefitArgs a) {
   }
 }
 
+// One lane per slot: its three corners gathered, and its frame from them.
 __global__ __launch_bounds__(kRefitBlock) void k_refit_tris(RefitArgs a) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kRefitBlock;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x; i < 3 * a.n_slots; i += stride) {
-    const float* p = a.positions + static_cast<uint64_t>(a.vidx[i]) * a.stride + a.offset;
-    float4 r = a.tris[i];
-    r.x = p[0];
-    r.y = p[1];
-    r.z = p[2];
-    a.tris[i] = r;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x; i < a.n_slots; i += stride) {
+    float4 r[3];
+    for (int k = 0; k < 3; k++) {
+      const float* p = a.positions + static_cast<uint64_t>(a.vidx[3 * i + k]) * a.stride + a.offset;
+      r[k] = make_float4(p[0], p[1], p[2], a.tris[3 * i + k].w);
+    }
+    for (int k = 0; k < 3; k++) a.tris[3 * i + k] = r[k];
+    float4 f[kFrameRows];
+    tri_frame(mk(r[0].x, r[0].y, r[0].z), mk(r[1].x, r[1].y, r[1].z), mk(r[2].x, r[2].y, r[2].z), f);
+    for (int k = 0; k < kFrameRows; k++) a.frames[kFrameRows * i + k] = f[k];
   }
+}
+
+__global__ __launch_bounds__(kRefitBlock) void k_tri_frames(const float4* tris, uint64_t n_slots, float4* frames) {
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x;
+  if (i >= n_slots) return;
+  float4 f[kFrameRows];
+  const float4 r0 = tris[3 * i], r1 = tris[3 * i + 1], r2 = tris[3 * i + 2];
+  tri_frame(mk(r0.x, r0.y, r0.z), mk(r1.x, r1.y, r1.z), mk(r2.x, r2.y, r2.z), f);
+  for (int k = 0; k < kFrameRows; k++) frames[kFrameRows * i + k] = f[k];
 }
 
 // Box of node i into the reference copy (floats 0..5 of the node) and its wide-node place.
@@ -280,11 +294,18 @@ hipError_t launch_export_nodes(const uint32_t* nodes, uint64_t n_nodes, const ui
   return hipGetLastError();
 }
 
+hipError_t launch_tri_frames(const float4* tris, uint64_t n_slots, float4* frames, hipStream_t s) {
+  if (n_slots)
+    hipLaunchKernelGGL(k_tri_frames, dim3(static_cast<uint32_t>((n_slots + kRefitBlock - 1) / kRefitBlock)),
+                       dim3(kRefitBlock), 0, s, tris, n_slots, frames);
+  return hipGetLastError();
+}
+
 hipError_t launch_refit(const RefitArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_refit_reset_bound, dim3(1), dim3(64), 0, s, a.coord_bound);
   hipLaunchKernelGGL(k_refit_bound, dim3(blocks_for(a.n_vertices) < kBoundBlocks ? blocks_for(a.n_vertices) : kBoundBlocks),
                      dim3(kRefitBlock), 0, s, a);
-  if (a.n_slots) hipLaunchKernelGGL(k_refit_tris, dim3(blocks_for(3 * a.n_slots)), dim3(kRefitBlock), 0, s, a);
+  if (a.n_slots) hipLaunchKernelGGL(k_refit_tris, dim3(blocks_for(a.n_slots)), dim3(kRefitBlock), 0, s, a);
   if (a.node_ids) {
     hipLaunchKernelGGL(k_refit_mark_clear, dim3(blocks_for(a.n_nodes)), dim3(kRefitBlock), 0, s, a.changed, a.n_nodes);
     if (a.n_ids) hipLaunchKernelGGL(k_refit_mark_ids, dim3(blocks_for(a.n_ids)), dim3(kRefitBlock), 0, s, a);
