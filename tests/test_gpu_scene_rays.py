@@ -1,0 +1,116 @@
+"""The scene raycast's four-lane kernel where its deferred decisions could go wrong: coincident instances
+(contenders past a lane's list, past a ray's row), rays it hands to the one-lane kernel, inverses that
+are not the matrices', grazing rays. The answer is that of the batched launch on every (ray, instance) pair."""
+import numpy as np
+import pytest
+
+import mbvh_amd as M
+from mbvh_amd import geometry as G, workloads as W
+from helpers import build_mesh
+from test_gpu_scene import GEOMS, _pairwise, _same
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = M.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="module")
+def meshes(ctx):
+    built = [build_mesh(f()) for f in GEOMS]
+    ms = [ctx.upload(t, g.positions, idx) for g, idx, t in built]
+    yield [b[0] for b in built], ms
+    for m in ms:
+        m.free()
+
+
+def _check(ctx, ms, w, **kw):
+    sc = ctx.scene(ms, w.matrix_world, w.matrix_world_inverse, w.instance_geometry)
+    got = sc.raycast_first(w.origins, w.directions, **kw)
+    ref = _pairwise(ctx, ms, w, None, **kw)
+    _same(got, ref)
+    sc.free()
+    return ref
+
+
+@pytest.mark.parametrize("copies", [2, 4, 5, 7, 40])
+def test_coincident_instances(ctx, meshes, copies):
+    geos, ms = meshes
+    w = W.scene_rays(geos, 3 * copies, 1500, seed=21)
+    for k in range(3 * copies):
+        for a in (w.matrix_world, w.matrix_world_inverse, w.instance_geometry):
+            a[k] = a[k // copies * copies]
+    ref = _check(ctx, ms, w)
+    hit = ref["instance"] != M.NO_HIT
+    assert hit.any() and np.all(ref["instance"][hit] % copies == 0)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65, 1000])
+def test_ray_counts(ctx, meshes, n):
+    geos, ms = meshes
+    _check(ctx, ms, W.scene_rays(geos, 9, n, seed=22))
+
+
+@pytest.mark.parametrize("kind", ["axis", "mixed", "unrotated"])
+def test_zero_direction_components(ctx, meshes, kind):
+    geos, ms = meshes
+    w = W.scene_rays(geos, 16, 1200, seed=23)
+    if kind == "unrotated":  # zero components only after the instance's transform
+        for k in range(16):
+            m = np.eye(4)
+            m[:3, 3] = w.matrix_world[k].reshape(4, 4).T[:3, 3]
+            w.matrix_world[k] = m.T.reshape(-1)
+            w.matrix_world_inverse[k] = np.linalg.inv(m).T.reshape(-1)
+    rows = slice(None) if kind == "axis" else slice(0, None, 3)
+    w.directions[rows] = np.eye(3, dtype=np.float32)[np.arange(1200) % 3][rows]
+    ctr = w.matrix_world.reshape(-1, 4, 4)[np.arange(1200) % 16, 3, :3]
+    w.origins[rows] = (ctr + 0.1 - 60 * w.directions)[rows]
+    assert (_check(ctx, ms, w)["face"][rows] != M.NO_HIT).any()
+
+
+@pytest.mark.parametrize("kind", ["shifted", "scaled", "projective", "sheared"])
+def test_any_inverse(ctx, meshes, kind):
+    geos, ms = meshes
+    w = W.scene_rays(geos, 12, 1500, seed=24, non_uniform=0.5)
+    inv = w.matrix_world_inverse
+    if kind == "shifted":
+        inv[:, 12:15] += 0.05
+    elif kind == "scaled":
+        inv[:, :15] *= np.float32(1.25)
+    elif kind == "projective":
+        inv[:, 15] = 1.0 + 1e-3
+        inv[:, 3] = 1e-4
+    else:
+        for k in range(12):
+            m = w.matrix_world[k].reshape(4, 4).T.astype(np.float64)
+            m[:3, :3] = m[:3, :3] @ np.array([[1, 0.9, 0], [0, 1, 0.4], [0, 0, 1]])
+            w.matrix_world[k] = m.T.reshape(-1)
+            inv[k] = np.linalg.inv(w.matrix_world[k].reshape(4, 4).astype(np.float64)).reshape(-1)
+    _check(ctx, ms, w, side=M.DOUBLE_SIDE)
+
+
+def test_grazing_rays(ctx):
+    """Rays in the plane of whole rows of triangles: undecided hits by the dozen."""
+    grid = np.arange(17, dtype=np.float32) / 4
+    x, y = np.meshgrid(grid, grid, indexing="ij")
+    pos = np.stack([x, y, 0 * x], -1).reshape(-1, 3)
+    a = (np.arange(16)[:, None] * 17 + np.arange(16)[None, :]).reshape(-1)
+    g0 = G.Geometry(pos, np.stack([a, a + 1, a + 17, a + 1, a + 18, a + 17], -1).reshape(-1).astype(np.uint16))
+    g, idx, tree = build_mesh(g0)
+    ms = [ctx.upload(tree, g.positions, idx)]
+    w = W.scene_rays([g], 6, 1024, seed=25)
+    rng = np.random.default_rng(26)
+    k = rng.integers(0, 6, 1024)
+    m = w.matrix_world.reshape(-1, 4, 4)[k].transpose(0, 2, 1).astype(np.float64)
+    p = np.concatenate([rng.uniform(0, 4, (1024, 2)), np.zeros((1024, 1))], 1)
+    q = np.concatenate([rng.uniform(-9, -5, (1024, 2)), 1e-6 * rng.standard_normal((1024, 1))], 1)
+    p, q = (np.einsum("nij,nj->ni", m[:, :3, :3], v) + m[:, :3, 3] for v in (p, q))
+    w.origins[:] = q
+    d = p - w.origins.astype(np.float64)
+    w.directions[:] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    _check(ctx, ms, w, side=M.DOUBLE_SIDE)
+    ms[0].free()

@@ -36,6 +36,11 @@ struct DeviceBuffer {
 // without that pass.
 constexpr uint64_t kHeavyCap = uint64_t{1} << 20;
 
+// Work-queue counters of the query kernels: one at the start, one for the list of long walks 128 bytes on,
+// and kWalkQueues from kWalkQueueOffset on, each on its own 128-byte line.
+constexpr size_t kWalkQueueOffset = 256;
+constexpr size_t kQueueBytes = kWalkQueueOffset + 128 * mbvh::kWalkQueues;
+
 struct mbvh_ctx {
   uint32_t magic = kCtxMagic;
   int device = 0;
@@ -51,6 +56,7 @@ struct mbvh_ctx {
   DeviceBuffer order;           // host-API query order
   DeviceBuffer order_ws;        // host-API ordering workspace
   DeviceBuffer heavy;           // queries left to a wave each (kHeavyCap entries, allocated with the context)
+  DeviceBuffer contenders;      // scene raycast: kSceneRow per ray of a launch (allocated with the first scene)
   DeviceBuffer hits[5];         // host-API all-hits results: offsets, face, dist, point, bary
   DeviceBuffer grad[11];        // host-API backward staging
   DeviceBuffer grad_ws;         // host-API backward workspace
@@ -131,6 +137,7 @@ struct mbvh_mesh {
   uint32_t* d_face_slot = nullptr;  // indirect meshes: face -> slot (0xFFFFFFFF if absent)
   float4* d_nodes4 = nullptr;       // 4-wide tree
   uint32_t* d_roots4 = nullptr;
+  uint32_t root4 = 0;               // the first root's 4-wide reference
   uint32_t max_stack4 = 0;
   uint64_t n_nodes = 0;
   uint32_t n_roots = 0;
@@ -551,7 +558,7 @@ extern "C" int mbvh_ctx_create(int32_t device, mbvh_ctx** out_ctx) {
     delete c;
     return set_error(MBVH_ERR_HIP, "mbvh_ctx_create: hipStreamCreate failed (%s)", hipGetErrorString(e));
   }
-  if (ensure_buffer(c->queue, 256)) {
+  if (ensure_buffer(c->queue, kQueueBytes)) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     return MBVH_ERR_OOM;
@@ -593,6 +600,7 @@ extern "C" void mbvh_ctx_destroy(mbvh_ctx* ctx) {
   if (ctx->grad_ws.ptr) (void)hipFree(ctx->grad_ws.ptr);
   if (ctx->order_ws.ptr) (void)hipFree(ctx->order_ws.ptr);
   if (ctx->heavy.ptr) (void)hipFree(ctx->heavy.ptr);
+  if (ctx->contenders.ptr) (void)hipFree(ctx->contenders.ptr);
   if (ctx->build_ws.ptr) (void)hipFree(ctx->build_ws.ptr);
   if (ctx->geo_ws.ptr) (void)hipFree(ctx->geo_ws.ptr);
   (void)hipStreamDestroy(ctx->stream);
@@ -753,6 +761,7 @@ extern "C" int mbvh_mesh_upload(mbvh_ctx* ctx, const void* const* roots, const u
   m->max_depth = max_depth;
   m->max_stack = max_stack;
   m->max_stack4 = max_stack4;
+  m->root4 = roots4[0];
   m->n_ref_nodes = maps.base;
   m->n_ref_leaves = maps.leaves.size();
   m->n_four_map = maps.four_map.size();
@@ -2886,6 +2895,8 @@ constexpr uint32_t kTlasMaxDepth = 24;
 // and the persistent waves of that pass.
 constexpr uint32_t kSceneHeavyBudget = 512;
 constexpr uint32_t kSceneWideWaves = 2048;
+// Threads over the rays the four-lane raycast leaves (usually none).
+constexpr uint64_t kSceneRestThreads = 1u << 17;
 
 struct mbvh_scene {
   uint32_t magic = 0x4E454353u;  // "SCEN"
@@ -2900,7 +2911,13 @@ struct mbvh_scene {
   uint32_t* d_geom = nullptr;
   uint32_t* d_tlas = nullptr;
   uint32_t* d_tlas_inst = nullptr;
+  float4* d_tlas4 = nullptr;       // the four-lane raycast's top level
+  uint2* d_tlas4_bigleaf = nullptr;
+  uint4* d_slots = nullptr;
+  uint32_t tlas4_root = 0;
+  float tlas_bound = 0.0f;
   uint32_t max_stack = 0;         // stack entries of the deepest instance walk (raycast)
+  uint32_t max_stack_rays4 = 0;   // the same for the four-lane raycast, the top level's entries below them
   uint32_t max_stack_points = 0;  // closest point: the top level's far children below them
   uint32_t max_stack_points4 = 0;  // the same for the four-lane kernel (4-wide instance trees)
   bool wide_ok = false;            // every instance tree's 4-wide walk fits the wave-per-point frontier
@@ -2955,7 +2972,7 @@ bool frame_inverse(const float* e, float* out) {
 
 void free_scene_buffers(mbvh_scene* sc) {
   void* bufs[] = {sc->d_meshes, sc->d_world, sc->d_inverse, sc->d_frame, sc->d_frame_ok, sc->d_geom, sc->d_tlas,
-                  sc->d_tlas_inst};
+                  sc->d_tlas_inst, sc->d_tlas4, sc->d_tlas4_bigleaf, sc->d_slots};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
 }
@@ -3088,16 +3105,101 @@ extern "C" int mbvh_scene_create(mbvh_ctx* ctx, const mbvh_mesh* const* meshes, 
   std::vector<uint32_t> slot_inst(std::max<uint32_t>(n_listed, 1), 0u);
   for (uint32_t s = 0; s < n_listed; s++) slot_inst[s] = listed[index[3ull * s] / 3];
 
+  // The four-lane raycast's top level: 4-wide, an instance per leaf where boxes can be told apart.
+  std::vector<float4> tlas4;
+  std::vector<uint2> tlas4_bigleaf;
+  std::vector<uint4> slots(kSceneSlotRows * std::max<size_t>(n_listed, 1), make_uint4(0u, 0u, 0u, 0u));
+  uint32_t tlas4_root = kDone4, tlas4_depth = 0;
+  float tlas_bound = 0.0f;
+  for (float v : prim_pos) tlas_bound = std::max(tlas_bound, std::fabs(v));
+  if (n_listed) {
+    for (uint32_t k = 0; k < 3 * n_listed; k++) index[k] = k;
+    const uint32_t range[2] = {0u, n_listed};
+    const mbvh_build_opts opts{MBVH_SAH, kTlasMaxDepth, 1, 0};
+    mbvh_tree* tree = nullptr;
+    if ((rc = mbvh_build(prim_pos.data(), 3ull * n_listed, 3, 0, index.data(), 4, index.size(), range, 1, &opts, &tree)))
+      return rc;
+    std::vector<WideNode> wide;
+    RefitMaps maps;
+    uint32_t root_ref = 0, depth = 0;
+    const NodeView v{tree->roots[0].data(), tree->roots[0].size() / kBytesPerNode};
+    rc = convert_root(v, n_listed, wide, tlas4_bigleaf, &root_ref, &depth, maps);
+    if (!rc) rc = build_bvh4(wide, root_ref, tlas4, &tlas4_root, &tlas4_depth, maps.four_map);
+    mbvh_tree_free(tree);
+    if (rc) return rc;
+    for (uint32_t s = 0; s < n_listed; s++) {
+      const uint32_t i = listed[index[3ull * s] / 3], g = instance_geometry[i];
+      const float* e = matrix_world + 16ull * i;
+      bool odd = false;
+      for (int k = 0; k < 3; k++) {
+        const float len2 = e[4 * k] * e[4 * k] + e[4 * k + 1] * e[4 * k + 1] + e[4 * k + 2] * e[4 * k + 2];
+        odd = odd || !(len2 > 1e-30f && len2 < 1e30f);
+      }
+      const uint64_t nodes_at = reinterpret_cast<uint64_t>(meshes[g]->d_nodes4);
+      const uint64_t bound_at = reinterpret_cast<uint64_t>(meshes[g]->d_coord_max);
+      uint4* rec = &slots[kSceneSlotRows * static_cast<size_t>(s)];
+      rec[0] = make_uint4(i, g, meshes[g]->root4, odd ? 1u : 0u);
+      rec[1] = make_uint4(static_cast<uint32_t>(nodes_at), static_cast<uint32_t>(nodes_at >> 32),
+                          static_cast<uint32_t>(bound_at), static_cast<uint32_t>(bound_at >> 32));
+      std::memcpy(rec + 2, matrix_world_inverse + 16ull * i, 64);
+      const uint64_t tris_at = reinterpret_cast<uint64_t>(meshes[g]->d_tris);
+      const float* v = matrix_world_inverse + 16ull * i;
+      const bool affine = v[3] == 0.0f && v[7] == 0.0f && v[11] == 0.0f && v[15] == 1.0f;
+      // W3 R3 = I and W3 r + w = 0 to 2^-20 of the magnitudes of their terms; those magnitudes
+      bool inverse = affine && !odd;
+      double norm = 0.0, cond = 0.0, shift = 0.0;
+      for (int row = 0; row < 3; row++) {
+        double tr = e[12 + row], tra = std::fabs(static_cast<double>(e[12 + row])), sums = 0.0;
+        for (int col = 0; col < 3; col++) {
+          double p = 0.0, pa = 0.0;
+          for (int k = 0; k < 3; k++) {
+            const double x = static_cast<double>(e[4 * k + row]) * v[4 * col + k];
+            p += x;
+            pa += std::fabs(x);
+          }
+          inverse = inverse && std::fabs(p - (row == col ? 1.0 : 0.0)) <= 9.5367431640625e-07 * pa;
+          sums += pa;
+          const double x = static_cast<double>(e[4 * col + row]) * v[12 + col];
+          tr += x;
+          tra += std::fabs(x);
+          norm += std::fabs(static_cast<double>(e[4 * col + row]));
+        }
+        inverse = inverse && std::fabs(tr) <= 9.5367431640625e-07 * tra;
+        cond = std::max(cond, sums);
+        shift = std::max(shift, tra);
+      }
+      // the norms of three rows: within 2 of the largest
+      const float mags[4] = {static_cast<float>(norm), static_cast<float>(cond * 2.0 * 3.814697265625e-06),
+                             static_cast<float>(shift * 2.0 * 3.814697265625e-06), 0.0f};
+      inverse = inverse && std::isfinite(mags[0]) && std::isfinite(mags[1]) && std::isfinite(mags[2]);
+      rec[6] = make_uint4(static_cast<uint32_t>(tris_at), static_cast<uint32_t>(tris_at >> 32), affine ? 1u : 0u,
+                          inverse ? 1u : 0u);
+      std::memcpy(rec + 7, mags, 16);
+    }
+  }
+  tlas4.resize(std::max<size_t>(tlas4.size(), 8), make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+  tlas4_bigleaf.resize(std::max<size_t>(tlas4_bigleaf.size(), 1), make_uint2(0u, 0u));
+  const uint32_t max_stack_rays4 = max_stack4 + 3 * tlas4_depth + 1;
+
   // closest point keeps the top level's far children (at most one per level) below the instance walks
   const uint32_t max_stack_points = max_stack + kTlasMaxDepth;
   const uint32_t max_stack_points4 = max_stack4 + kTlasMaxDepth;
-  if ((rc = reserve_stack(ctx, std::max(max_stack_points, max_stack_points4)))) return rc;
+  if ((rc = reserve_stack(ctx, std::max(max_stack_rays4, std::max(max_stack_points, max_stack_points4))))) return rc;
+  // the raycast's rows, here so that the device-pointer entry points allocate nothing (without them
+  // it takes one lane per ray)
+  if (ensure_buffer(ctx->contenders, (kHeavyCap * kSceneRow + kScenePool) * sizeof(uint2))) {
+    ctx->contenders = DeviceBuffer{};
+    clear_error();
+  }
   mbvh_scene* sc = new (std::nothrow) mbvh_scene();
   if (!sc) return set_error(MBVH_ERR_OOM, "%s: out of host memory", fn);
   sc->ctx = ctx;
   sc->n_meshes = n_meshes;
   sc->n_instances = n_instances;
   sc->max_stack = max_stack;
+  sc->max_stack_rays4 = max_stack_rays4;
+  sc->tlas4_root = tlas4_root;
+  sc->tlas_bound = tlas_bound;
   sc->max_stack_points = max_stack_points;
   sc->max_stack_points4 = max_stack_points4;
   sc->wide_ok = 64ull * (max_stack4 > 0 ? max_stack4 - 1 : 0) + 256 <= kWideFrontier;
@@ -3128,6 +3230,13 @@ extern "C" int mbvh_scene_create(mbvh_ctx* ctx, const mbvh_mesh* const* meshes, 
   }
   if (e == hipSuccess) e = hipMemcpy(sc->d_tlas, nodes.data(), nodes.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(sc->d_tlas_inst, slot_inst.data(), slot_inst.size() * 4, hipMemcpyHostToDevice);
+  auto put = [&](auto** dst, const auto& src) {
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(dst), src.size() * sizeof(src[0]));
+    if (e == hipSuccess) e = hipMemcpy(*dst, src.data(), src.size() * sizeof(src[0]), hipMemcpyHostToDevice);
+  };
+  put(&sc->d_tlas4, tlas4);
+  put(&sc->d_tlas4_bigleaf, tlas4_bigleaf);
+  put(&sc->d_slots, slots);
   if (e != hipSuccess) {
     free_scene_buffers(sc);
     delete sc;
@@ -3453,9 +3562,41 @@ int enqueue_scene(mbvh_ctx* ctx, const mbvh_scene* sc, const float* o, const flo
   a.out_dist = dist;
   a.out_point = point;
   a.out_bary = bary;
-  const uint64_t threads = launch_threads(n, ctx->max_threads);
-  a.stack = stack_of(ctx, threads);
-  MBVH_HIP(launch_scene_raycast_first(a, threads, s));
+  if (!ctx->heavy.ptr || !ctx->contenders.ptr || sc->max_stack_rays4 > kMinLdsStack + ctx->stack_ovf_entries) {
+    const uint64_t threads = launch_threads(n, ctx->max_threads);
+    a.stack = stack_of(ctx, threads);
+    MBVH_HIP(launch_scene_raycast_first(a, threads, s));
+    return MBVH_OK;
+  }
+  a.tlas4 = sc->d_tlas4;
+  a.tlas4_root = sc->tlas4_root;
+  a.tlas4_bigleaf = sc->d_tlas4_bigleaf;
+  a.slots = sc->d_slots;
+  a.contenders = static_cast<uint2*>(ctx->contenders.ptr);
+  a.contender_pool = a.contenders + kHeavyCap * kSceneRow;
+  a.contender_pool_count = static_cast<uint32_t*>(ctx->queue.ptr) + 16;  // beside the long walks' counter's line
+  a.contender_pool_cap = kScenePool;
+  a.tlas_bound = sc->tlas_bound;
+  a.queue = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->queue.ptr) + kWalkQueueOffset);
+  a.heavy = static_cast<uint32_t*>(ctx->heavy.ptr);
+  a.heavy_count = static_cast<uint32_t*>(ctx->queue.ptr) + 32;
+  // as many rays at a time as the list of those left to the one-lane kernel holds
+  for (uint64_t at = 0; at < n; at += kHeavyCap) {
+    a.n = std::min(kHeavyCap, n - at);
+    a.origins = o + 3 * at;
+    a.directions = d + 3 * at;
+    a.out_face = face + at;
+    a.out_instance = inst ? inst + at : nullptr;
+    a.out_dist = dist ? dist + at : nullptr;
+    a.out_point = point ? point + 3 * at : nullptr;
+    a.out_bary = bary ? bary + 3 * at : nullptr;
+    const uint64_t quads = launch_threads(4 * a.n, ctx->max_threads) / 4;
+    a.stack = stack_of(ctx, quads);
+    MBVH_HIP(launch_scene_raycast_first4(a, quads, s));
+    const uint64_t threads = launch_threads(std::min<uint64_t>(a.n, kSceneRestThreads), ctx->max_threads);
+    a.stack = stack_of(ctx, threads);
+    MBVH_HIP(launch_scene_raycast_first(a, threads, s));
+  }
   return MBVH_OK;
 }
 

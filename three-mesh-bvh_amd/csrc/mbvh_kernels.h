@@ -265,12 +265,30 @@ struct BatchArgs {
   StackScratch stack;
 };
 
+constexpr uint32_t kSceneRow = 4;       // contenders of a ray before it takes a row of the pool
+constexpr uint32_t kScenePool = 1u << 20;  // pool entries per launch; when they are gone, the one-lane kernel
+constexpr uint32_t kSceneSlotRows = 8;  // uint4 per top-level slot
 // Scene: closest first hit over instances, one launch (TLAS over the instances' world boxes).
 struct SceneArgs {
   const MeshView* meshes;
   uint32_t n_meshes;
   const uint32_t* tlas;            // reference-format nodes (8 words) over the instances' world boxes
   const uint32_t* tlas_inst;       // instance at each TLAS primitive slot
+  // the four-lane raycast's top level: a 4-wide tree (MeshView's nodes4 layout) with one instance per
+  // leaf, its root reference, large leaves, and the largest |coordinate| of its boxes
+  const float4* tlas4;
+  uint32_t tlas4_root;
+  const uint2* tlas4_bigleaf;
+  float tlas_bound;
+  // per slot of that tree: (instance, mesh, the mesh's first 4-wide root, whether a column of matrixWorld
+  // has no finite positive length), (nodes4, coord_max: device addresses), the caller's inverse (4 rows), (tris: device
+  // address, whether that inverse is affine, whether it is matrixWorld's to 2^-20), the magnitudes of their
+  // products (sum of |W3|; 2^-18 times the largest row sum of |W3| |R3|; 2^-18 times that of the translations)
+  const uint4* slots;
+  uint2* contenders;               // kSceneRow (triangle slot, instance) per ray, ended by kNoHit when fewer
+  uint2* contender_pool;           // rows of the rays with more
+  uint32_t* contender_pool_count;
+  uint32_t contender_pool_cap;
   const float* world;              // 16 floats per instance (local -> world, column-major)
   const float* inverse;            // 16 floats per instance (world -> local)
   // closest point's box bounds in the instance frame: 16 floats per instance, the float rounding of
@@ -292,14 +310,20 @@ struct SceneArgs {
   float* out_bary;
   StackScratch stack;
   const uint32_t* order;           // closest point: visit order of the points (NULL: 0..n-1)
-  uint32_t* queue;                 // closest point, four lanes: work-queue counter
+  uint32_t* queue;                 // four lanes: work-queue counter (raycast: kWalkQueues, 128 bytes apart)
   // closest point, four lanes: a point still unfinished after `heavy_budget` leaf steps is left to
-  // the wave-per-point pass, its index appended to `heavy` (count in heavy_count); heavy NULL: none
+  // the wave-per-point pass, its index appended to `heavy` (count in heavy_count); heavy NULL: none.
+  // Raycast, four lanes: the rays left to the one-lane kernel
   uint32_t* heavy;
   uint32_t* heavy_count;
   uint32_t heavy_budget;
 };
+// One lane per ray, over a.heavy (*a.heavy_count rays) or, when it is NULL, every ray.
 hipError_t launch_scene_raycast_first(const SceneArgs& a, uint64_t threads, hipStream_t s);
+// Four lanes per ray (quads: rays traced at once, a multiple of 64; a.n < 2^32) and the resolution of
+// their contenders; the rays it leaves are listed in a.heavy, which must hold a.n entries.
+constexpr uint32_t kWalkQueues = 8;  // one per XCD
+hipError_t launch_scene_raycast_first4(const SceneArgs& a, uint64_t quads, hipStream_t s);
 // Closest point over the instances: `origins` holds the world points (directions, side, near / far unused).
 hipError_t launch_scene_closest_point(const SceneArgs& a, uint64_t threads, hipStream_t s);
 // The same with four lanes per point (threads = 4 per point, a multiple of the block; a work queue).

@@ -140,6 +140,8 @@ __device__ __forceinline__ Tri load_tri(const float4* tris, uint32_t slot) {
 // origin) ignored, hit iff max(entries) <= min(exits) && entry <= far && exit >= near. The FP32
 // interval is widened by a few ulps so a box the exact ray touches is never rejected.
 // ------------------------------------------------------------------------------------------
+__device__ __forceinline__ float rcp_approx(float x) { return __builtin_amdgcn_rcpf(x); }
+
 struct RayBox {
   float ox, oy, oz;
   float ix, iy, iz;  // 1 / direction
@@ -403,9 +405,27 @@ __device__ __forceinline__ int hit_fast(f3 o, f3 d, float dlen, const RayBand& b
   return kHit;
 }
 
+// A lower bound of the ray parameter of a hit that is not decided (if there is one it is inside the
+// triangle's box): entry distance of the box, widened like any box's. A ray along a surface is
+// undecided for whole rows of triangles; without the bound every one of them stays a candidate.
+__device__ __forceinline__ float unsure_from(const RayBox4& rb, const Tri& t) {
+  float lb;
+  slab4(rb, make_float4(fminf(fminf(t.p0.x, t.p1.x), t.p2.x), fminf(fminf(t.p0.y, t.p1.y), t.p2.y),
+                        fminf(fminf(t.p0.z, t.p1.z), t.p2.z), fmaxf(fmaxf(t.p0.x, t.p1.x), t.p2.x)),
+        make_float4(fmaxf(fmaxf(t.p0.y, t.p1.y), t.p2.y), fmaxf(fmaxf(t.p0.z, t.p1.z), t.p2.z), 0.0f, 0.0f), 0.0f, kInf, lb);
+  return lb;
+}
+__device__ __forceinline__ float unsure_from(const RayBox& rb, const Tri& t) {
+  float lb;
+  slab(rb, fminf(fminf(t.p0.x, t.p1.x), t.p2.x), fminf(fminf(t.p0.y, t.p1.y), t.p2.y),
+       fminf(fminf(t.p0.z, t.p1.z), t.p2.z), fmaxf(fmaxf(t.p0.x, t.p1.x), t.p2.x), fmaxf(fmaxf(t.p0.y, t.p1.y), t.p2.y),
+       fmaxf(fmaxf(t.p0.z, t.p1.z), t.p2.z), 0.0f, kInf, lb);
+  return lb;
+}
+
 // ------------------------------------------------------------------------------------------
 // Candidate list (per lane, in visit order). `lb` is a lower bound of the candidate's exact key
-// (ray parameter or squared distance); -inf marks a candidate whose hit/miss is undecided. A
+// (ray parameter or squared distance), also of one whose hit is undecided. A
 // candidate whose lb exceeds the best upper bound U can never win and is dropped.
 // ------------------------------------------------------------------------------------------
 struct Cands {
@@ -733,12 +753,11 @@ __device__ __forceinline__ FirstHit trace_first(const MeshView& M, StackT& st, u
             et = 2.0f * kU * t;
           }
           if (res == kMiss) continue;
-          if (res == kHit) {
-            hits++;
-            const float lb = t - et;
-            if (lb > U) continue;  // certainly behind a known hit
-            U = fminf(U, t + et);
-          }
+          float lb = t - et;
+          if (res == kUnsure) lb = unsure_from(rb, tr);
+          if (res == kHit) hits++;
+          if (lb > U) continue;  // certainly behind a known hit
+          if (res == kHit) U = fminf(U, t + et);
           if (cl.n == kCand && !cl.compact(U)) {
             // full of live candidates: settle them now and keep the winner
             const Winner r = resolve_ray<kLo, false>(cl, U, o, d, ol, dl, M.tris, tie_tree(M), side_mask, win);
@@ -751,7 +770,7 @@ __device__ __forceinline__ FirstHit trace_first(const MeshView& M, StackT& st, u
               cl.n = 1;
             }
           }
-          cl.put(cl.n++, s, res == kHit ? t - et : -kInf);
+          cl.put(cl.n++, s, lb);
         }
         ref = kDone;
         while (st.sp > 0) {
@@ -846,6 +865,13 @@ __device__ __forceinline__ T quad_xor2(T v) {  // lanes 2 3 0 1
   return quad_dpp<0x4E>(v);
 }
 
+__device__ __forceinline__ bool quad_any(bool v) {
+  uint32_t u = v ? 1u : 0u;
+  u |= quad_xor1(u);
+  u |= quad_xor2(u);
+  return u != 0u;
+}
+
 // One node step of a quad: lane q holds child q of the node, `in` saying whether it is entered,
 // with its key (entry t or box score, a lower bound) and ref. The entered children are ranked by
 // their key (the order only steers the search, any order gives the same result): the key's bits,
@@ -854,7 +880,8 @@ __device__ __forceinline__ T quad_xor2(T v) {  // lanes 2 3 0 1
 // entered child is written by its own lane onto the quad stack, farthest deepest, so that pops come
 // nearest first; the stack keeps the exact key. Sets `overflow` (and returns kDone) when the stack
 // cannot take them.
-__device__ __forceinline__ uint32_t quad_children(QuadStack& st, uint32_t lane, bool in, float key, uint32_t cref,
+template <typename StackT>
+__device__ __forceinline__ uint32_t quad_children(StackT& st, uint32_t lane, bool in, float key, uint32_t cref,
                                                   bool& overflow) {
   const uint32_t q = lane & 3u;
   const uint32_t kb = __float_as_uint(key);
@@ -937,10 +964,10 @@ __device__ __forceinline__ FirstHit trace_first4(const MeshView& M, QuadStack& s
           float t = 0.0f, et = 0.0f;
           const int res = hit_fast<kLo>(o, d, dlen, band, tr, mask, near_dist, far_dist, t, et);
           if (res == kMiss) continue;
-          if (res == kHit) {
-            if (t - et > Ul) continue;  // certainly behind a known hit
-            Ul = fminf(Ul, t + et);
-          }
+          float lb = t - et;
+          if (res == kUnsure) lb = unsure_from(rb, tr);
+          if (lb > Ul) continue;  // certainly behind a known hit
+          if (res == kHit) Ul = fminf(Ul, t + et);
           if (cl.n == kCand && !cl.compact(Ul)) {
             const Winner r = resolve_ray<kLo, true>(cl, Ul, o, d, ol, dl, M.tris, T, side_mask, win);
             const uint32_t w = r.w;
@@ -952,7 +979,7 @@ __device__ __forceinline__ FirstHit trace_first4(const MeshView& M, QuadStack& s
               cl.n = 1;
             }
           }
-          cl.put(cl.n++, s, res == kHit ? t - et : -kInf);
+          cl.put(cl.n++, s, lb);
         }
         Ul = fminf(Ul, quad_xor1(Ul));
         U = fminf(Ul, quad_xor2(Ul));
@@ -1422,7 +1449,6 @@ __global__ __launch_bounds__(kBlock) void k_raycast_all(RaycastAllArgs A) {
 // divisions use the hardware reciprocal (1 ulp) and the face region clamps the three sub-areas at
 // 0: every branch returns a convex combination of a, b, c with weights valid to a few ulps.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ float rcp_approx(float x) { return __builtin_amdgcn_rcpf(x); }
 
 __device__ __forceinline__ f3 closest_on_triangle(f3 p, f3 a, f3 b, f3 c) {
   const f3 ab = sub(b, a), ac = sub(c, a), ap = sub(p, a);
@@ -2282,7 +2308,8 @@ __device__ __forceinline__ bool box_entry(f3 o, f3 inv, const float* b, float ne
   return tmin <= tmax && tmax >= near_dist;
 }
 
-// One lane per ray. The TLAS (reference node format over the instances' world boxes, expanded
+// One lane per ray, for the rays the four-lane kernel left (A.heavy lists them; NULL: every ray). The
+// TLAS (reference node format over the instances' world boxes, expanded
 // outward when built) is walked near child first and pruned by the best world distance so far
 // (with a 2^-16 relative margin: box distances and hit distances round differently); each
 // instance leaf brings the ray into the instance's frame and traces its mesh exactly as the batched
@@ -2304,7 +2331,9 @@ __global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
   st.capacity = 8 + static_cast<int>(A.stack.ovf_entries);
   const float qnan = __int_as_float(0x7fc00000);
   const float margin = 1.0f + 1.0f / 65536.0f;
-  for (uint64_t ray = gtid; ray < A.n; ray += static_cast<uint64_t>(gridDim.x) * kBlock) {
+  const uint64_t count = A.heavy ? static_cast<uint64_t>(*A.heavy_count) : A.n;
+  for (uint64_t k = gtid; k < count; k += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const uint64_t ray = A.heavy ? A.heavy[k] : k;
     const f3 ow = mk(A.origins[3 * ray], A.origins[3 * ray + 1], A.origins[3 * ray + 2]);
     const f3 dw = mk(A.directions[3 * ray], A.directions[3 * ray + 1], A.directions[3 * ray + 2]);
     const f3 iw = mk(1.0f / dw.x, 1.0f / dw.y, 1.0f / dw.z);
@@ -2379,6 +2408,506 @@ __global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
       A.out_bary[3 * ray + 1] = best.bary.y;
       A.out_bary[3 * ray + 2] = best.bary.z;
     }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// Scene first hit, four lanes per ray, one loop for both levels. A quad of lanes traces one ray: in the
+// top level (a 4-wide tree over the instances' world boxes) and in the instances' 4-wide trees the
+// same node step scores four children, ranks and pushes them (quad_children); a leaf's triangles are
+// split over the lanes. The sixteen quads of a wave are in different places, so the wave steps by
+// majority: each round runs the step (nodes, triangles, or a switch of levels) that most of its live
+// quads are at. A quad whose ray is finished takes another from the wave's batch once kSceneRefill
+// quads are; batches come from one queue per XCD.
+//
+// Nothing is settled exactly here. On leaving an instance the ray's hit there has its parameter within
+// [least lower bound, U], so its world distance (the float the answer reports, from the rounded hit
+// point through the instance's matrix) is within an interval: with p(t) = o + t d in the instance's
+// frame, W p(t) = ow + delta + t W3 d, delta = W o - ow (small when the caller's inverse is W's; any
+// inverse gives a valid interval), so the distance is t |W3 d| within |delta| plus the roundings, at
+// most 2^-19 of the magnitudes involved. An instance whose interval is past the contenders' least upper
+// end is dropped, one wholly before theirs replaces them, otherwise its candidates join them.
+// k_scene_ray_resolve settles each ray's contenders (nearly always one triangle) as the one-lane kernel does:
+// per instance the exact first hit with the reference's tie rule, then the least world distance,
+// equal ones to the lower instance. Rays with a zero direction component, in the world or in an
+// instance they reach, and rays with more contenders than a row holds go to the one-lane kernel
+// (A.heavy lists them).
+//
+// What bounds it: vector issue (1.5 of 2.0 ms for 512 instances and 2^20 rays from outside; about 20
+// node, 4 triangle and 5 switch steps per ray, half the lanes busy) at four waves per SIMD (126
+// registers; 96 spill and are slower). One lane per ray with each instance's walk nested in the top
+// level's and settled exactly on the way kept 3% of the lanes busy: 7.9 -> 2.1 ms. On the way: popping
+// one entry per step instead of looping to the next live one, no exact step in this kernel (each in a
+// quarter of its lanes), instance records in one load, each step in a loop of its own (a third fewer
+// instructions, the rest being copies of the walk's state).
+// ------------------------------------------------------------------------------------------
+constexpr int kSceneRefill = 3;           // 2 and 6 measured 1 and 2% slower
+constexpr int kSceneLds = 32;             // stack entries per quad in LDS
+constexpr uint32_t kSceneBatch = 64;
+constexpr uint32_t kPooled = 0xFFFFFFFDu;  // a row's first word: its contenders are in the pool
+constexpr int kContend = 4;               // contenders per lane
+
+// ray_box4 for the scene's quads: the reciprocals by the hardware's 1-ulp instruction. That is u more
+// relative error than a division on both plane products, 6 u S of the widening's 8 u S. False: a zero
+// direction component or constants that are not finite (literal_ray).
+__device__ __forceinline__ bool scene_box4(f3 o, f3 d, float coord_max, RayBox4& r) {
+  r.ix = rcp_approx(d.x);
+  r.iy = rcp_approx(d.y);
+  r.iz = rcp_approx(d.z);
+  const float ox = -o.x * r.ix, oy = -o.y * r.iy, oz = -o.z * r.iz;
+  const float ex = 8.0f * kU * ((coord_max + fabsf(o.x)) * fabsf(r.ix));
+  const float ey = 8.0f * kU * ((coord_max + fabsf(o.y)) * fabsf(r.iy));
+  const float ez = 8.0f * kU * ((coord_max + fabsf(o.z)) * fabsf(r.iz));
+  r.lx = ox - ex;
+  r.ly = oy - ey;
+  r.lz = oz - ez;
+  r.hx = ox + ex;
+  r.hy = oy + ey;
+  r.hz = oz + ez;
+  r.sx = r.ix >= 0.0f;
+  r.sy = r.iy >= 0.0f;
+  r.sz = r.iz >= 0.0f;
+  // a sub-2^-126 reciprocal is flushed to zero: |d| that large is left to the one-lane kernel too
+  const float big = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+  return fabsf(r.ix) + fabsf(r.iy) + fabsf(r.iz) + fabsf(ox) + fabsf(oy) + fabsf(oz) + ex + ey + ez < kInf && big < 1e30f;
+}
+
+// The terms of a ray's world distance in an instance's frame: t * along within off + t * grow. From the
+// matrices (any inverse); where the caller's inverse is W's to 2^-20, the kernel takes |W3 d| as
+// |dw| / |inverse dw| and W o as ow, with the products' magnitudes (from the scene's creation) times 2^-18
+// in the bounds.
+struct WorldSpan {
+  float along, off, grow;
+};
+__device__ __forceinline__ WorldSpan world_span(const float* W, f3 ow, f3 o, f3 d) {
+  const float4* w4 = reinterpret_cast<const float4*>(W);
+  const float4 a = w4[0], b = w4[1], c = w4[2], t = w4[3];
+  const f3 along = mk(a.x * d.x + b.x * d.y + c.x * d.z, a.y * d.x + b.y * d.y + c.y * d.z,
+                      a.z * d.x + b.z * d.y + c.z * d.z);
+  const f3 delta = mk(a.x * o.x + b.x * o.y + c.x * o.z + t.x - ow.x, a.y * o.x + b.y * o.y + c.y * o.z + t.y - ow.y,
+                      a.z * o.x + b.z * o.y + c.z * o.z + t.z - ow.z);
+  const float norm = fabsf(a.x) + fabsf(a.y) + fabsf(a.z) + fabsf(b.x) + fabsf(b.y) + fabsf(b.z) + fabsf(c.x) +
+                     fabsf(c.y) + fabsf(c.z);
+  constexpr float kRound = 1.0f / 524288.0f;  // 2^-19
+  WorldSpan s;
+  s.along = __builtin_amdgcn_sqrtf(dot(along, along));
+  s.off = __builtin_amdgcn_sqrtf(dot(delta, delta)) * (1.0f + kRound) +
+          kRound * (norm * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z)) + fabsf(t.x) + fabsf(t.y) + fabsf(t.z) + fabsf(ow.x) +
+                    fabsf(ow.y) + fabsf(ow.z));
+  s.grow = kRound * norm * (fabsf(d.x) + fabsf(d.y) + fabsf(d.z));
+  return s;
+}
+
+// A quad's stack with kSceneLds entries in LDS.
+struct SceneStack {
+  uint2* lds;
+  uint2* ovf;
+  uint64_t ovf_stride;
+  uint64_t gquad;
+  uint32_t qid;
+  int capacity;
+  int sp;
+  __device__ __forceinline__ void put(int pos, uint32_t ref, uint32_t aux) {
+    if (pos < kSceneLds)
+      lds_store(lds, pos * (kBlock / 4) + qid, make_uint2(ref, aux));
+    else
+      ovf_store(ovf, static_cast<uint64_t>(pos - kSceneLds) * ovf_stride + gquad, make_uint2(ref, aux));
+  }
+  __device__ __forceinline__ uint2 pop() {
+    const int pos = --sp;
+    if (pos < kSceneLds) return lds_load(lds, pos * (kBlock / 4) + qid);
+    return ovf_load(ovf, static_cast<uint64_t>(pos - kSceneLds) * ovf_stride + gquad);
+  }
+};
+
+__global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A) {
+  __shared__ uint2 qstack[kSceneLds * (kBlock / 4)];
+  __shared__ uint2 contend[kContend * kBlock];  // (slot, instance)
+  __shared__ float4 wbox[2 * (kBlock / 4)];
+  __shared__ float wbox_hz[kBlock / 4];
+  const uint32_t lane = threadIdx.x, wl = lane & 63u, q4 = lane & 3u, qid = lane >> 2;
+  SceneStack st;
+  st.lds = qstack;
+  st.ovf = A.stack.ovf;
+  st.ovf_stride = static_cast<uint64_t>(gridDim.x) * (kBlock / 4);
+  st.gquad = static_cast<uint64_t>(blockIdx.x) * (kBlock / 4) + qid;
+  st.qid = qid;
+  st.capacity = kSceneLds + static_cast<int>(A.stack.ovf_entries);
+  st.sp = 0;
+  const uint32_t n = static_cast<uint32_t>(A.n);
+  const uint32_t batches = (n + kSceneBatch - 1) / kSceneBatch, share = (batches + kWalkQueues - 1) / kWalkQueues;
+  uint32_t cur = 0, end = 0, home = blockIdx.x % kWalkQueues, tried = 0;
+  const f3 z = mk(0.0f, 0.0f, 0.0f);
+  const bool window = A.near_dist > 0.0f || A.far_dist < kInf;
+
+  // The quad's ray and walk. inst: the instance being walked (kNoHit: the top level); [s, e) its
+  // leaf's triangles, or the top-level leaf's slots (kept in [ts, te) during an instance).
+  bool live = false, give_up = false;
+  uint32_t ray = kNoHit, inst = kNoHit, ref = kDone, s = 0, e = 0, ts = 0, te = 0, root = 0;
+  int base = 0;
+  const float4* nodes = A.tlas4;
+  const float4* tris = nullptr;
+  const MeshView* mesh = A.meshes;
+  f3 o = z, d = z;
+  RayBox4 rb = {};
+  float U = kInf, near_t = 0.0f, far_t = kInf;
+  Cands cl;
+  cl.lane = lane;
+  cl.n = 0;
+  int held = 0;                               // this lane's contenders
+  float best_lo = kInf, best_hi = kInf;       // the contenders' world distances
+
+  float wlen = 1.0f;                          // length of the world direction
+  WorldSpan span = {};                        // of the instance being walked
+  // The top level's ray (its box constants kept in LDS) and bound.
+  auto to_top = [&]() {
+    const float4 a = wbox[qid], b = wbox[kBlock / 4 + qid];
+    rb.ix = a.x;
+    rb.iy = a.y;
+    rb.iz = a.z;
+    rb.lx = a.w;
+    rb.ly = b.x;
+    rb.lz = b.y;
+    rb.hx = b.z;
+    rb.hy = b.w;
+    rb.hz = wbox_hz[qid];
+    rb.sx = rb.ix >= 0.0f;
+    rb.sy = rb.iy >= 0.0f;
+    rb.sz = rb.iz >= 0.0f;
+    constexpr float kMargin = 1.0f / 65536.0f;
+    const float per = rcp_approx(wlen);
+    U = fminf(best_hi, A.far_dist) * per * (1.0f + kMargin) + 1e-30f;
+    near_t = A.near_dist * per * (1.0f - kMargin);
+    far_t = kInf;
+    nodes = A.tlas4;
+    inst = kNoHit;
+    s = ts;
+    e = te;
+    base = 0;
+  };
+  // Ends a step: a quad with nothing in hand pops one entry (past the bound it pops again in the next
+  // node step, so that no quad waits for another's pops), a leaf's range is taken, and a ray whose top
+  // level is exhausted is finished. A quad is then at a node (ref), at triangles (s < e), popping, or
+  // at a switch of levels: an instance exhausted, or instances to enter (s < e in the top level).
+  auto settle = [&]() {
+    if (ref == kDone && s >= e && st.sp > base) {
+      const uint2 p = st.pop();
+      if (__uint_as_float(p.y) <= U) ref = p.x;
+    }
+    if (ref & kRefLeaf) {
+      uint32_t f, c;
+      leaf_range(ref, inst == kNoHit ? A.tlas4_bigleaf : mesh->bigleaf, f, c);
+      ref = kDone;
+      s = f;
+      e = f + c;
+    }
+    if (inst == kNoHit && ref == kDone && s >= e && st.sp == 0) live = false;
+  };
+
+  while (true) {
+    const uint64_t lm = __ballot(live);
+    const int idle = (64 - __popcll(lm)) >> 2;
+    if (idle == 16 || (idle >= kSceneRefill && (tried < kWalkQueues || cur < end))) {
+      // ---- the finished rays' contenders, then new rays ----
+      if (!live && ray != kNoHit) {
+        const uint32_t h = static_cast<uint32_t>(held);
+        const uint32_t h0 = quad_bcast<0>(h), h1 = quad_bcast<1>(h), h2 = quad_bcast<2>(h), h3 = quad_bcast<3>(h);
+        const uint32_t total = h0 + h1 + h2 + h3;
+        uint2* const row = A.contenders + static_cast<uint64_t>(kSceneRow) * ray;
+        uint2* to = row;
+        if (!give_up && total > kSceneRow) {  // a row of the pool, named in the ray's own
+          uint32_t at = 0;
+          if (q4 == 0) at = atomicAdd(A.contender_pool_count, total);
+          at = quad_bcast<0>(at);
+          give_up = at > A.contender_pool_cap || A.contender_pool_cap - at < total;
+          to = A.contender_pool + at;
+          if (q4 == 0 && !give_up) {
+            row[0] = make_uint2(kPooled, at);
+            row[1] = make_uint2(total, 0u);
+          }
+        }
+        if (give_up) {
+          if (q4 == 0) {
+            A.heavy[atomicAdd(A.heavy_count, 1u)] = ray;
+            row[0] = make_uint2(kOverflow, 0u);  // not for the resolution
+          }
+        } else {
+          uint32_t at = q4 == 0 ? 0u : (q4 == 1 ? h0 : (q4 == 2 ? h0 + h1 : h0 + h1 + h2));
+          for (uint32_t i = 0; i < h; i++) to[at++] = contend[i * kBlock + lane];
+          if (q4 == 3 && total < kSceneRow) row[total] = make_uint2(kNoHit, 0u);
+        }
+        ray = kNoHit;
+      }
+      while (cur == end && tried < kWalkQueues) {
+        uint32_t b = 0;
+        if (wl == 0) b = atomicAdd(A.queue + 32 * home, 1u);
+        b = __builtin_amdgcn_readfirstlane(b);
+        const uint32_t at = home * share + b;
+        if (b < share && at < batches) {
+          cur = at * kSceneBatch;
+          end = min(cur + kSceneBatch, n);
+        } else {
+          home = (home + 1) % kWalkQueues;
+          tried++;
+        }
+      }
+      if (cur == end && idle == 16) break;  // every wave reaches this exit: the queues only run empty
+      const uint32_t take = min(end - cur, static_cast<uint32_t>(idle));
+      const uint64_t below = ~lm & ((1ull << (wl & ~3u)) - 1ull);  // idle lanes of the quads below this one
+      const uint32_t rank = static_cast<uint32_t>(__popcll(below)) >> 2;
+      if (!live && rank < take) {
+        ray = cur + rank;
+        best_lo = best_hi = kInf;
+        held = cl.n = 0;
+        ts = te = 0;
+        st.sp = 0;
+        const f3 ow = load3(A.origins, ray), dw = load3(A.directions, ray);
+        wlen = __builtin_amdgcn_sqrtf(dot(dw, dw));
+        give_up = !scene_box4(ow, dw, A.tlas_bound, rb);
+        // the quad's own entries, written alike by its four lanes
+        wbox[qid] = make_float4(rb.ix, rb.iy, rb.iz, rb.lx);
+        wbox[kBlock / 4 + qid] = make_float4(rb.ly, rb.lz, rb.hx, rb.hy);
+        wbox_hz[qid] = rb.hz;
+        to_top();
+        ref = A.tlas4_root;
+        live = !give_up;
+        if (live) settle();
+      }
+      cur += take;
+      continue;
+    }
+    // Each step repeats while its quads are the most of those live and no refill is due (a loop of
+    // its own keeps the rest of the walk's state in place).
+    const bool more = tried < kWalkQueues || cur < end;
+    auto at_node = [&]() { return live && (ref != kDone || (s >= e && st.sp > base)); };
+    auto at_tris = [&]() { return live && ref == kDone && inst != kNoHit && s < e; };
+    while (true) {
+      const int nl = __popcll(__ballot(live)), nn = __popcll(__ballot(at_node())), nt = __popcll(__ballot(at_tris()));
+      if (nn == 0 || nn < nt || nn < nl - nn - nt || (more && nl <= 4 * (16 - kSceneRefill))) break;
+      const bool mine = at_node();
+      if (mine && ref == kDone) settle();
+      if (mine && ref != kDone && live) {
+        // ---- node step ----
+        const float4 c0 = nodes[8ull * ref + 2 * q4];
+        const float4 c1 = nodes[8ull * ref + 2 * q4 + 1];
+        const uint32_t cref = __float_as_uint(c1.z);
+        float t;
+        const bool box = slab4(rb, c0, c1, near_t, far_t, t);
+        bool overflow = false;
+        ref = quad_children(st, lane, (cref != kDone) & box & (t <= U), t, cref, overflow);
+        if (overflow) {
+          give_up = true;  // the one-lane kernel reports it
+          live = false;
+        } else {
+          settle();
+        }
+      }
+    }
+    while (true) {
+      const int nl = __popcll(__ballot(live)), nn = __popcll(__ballot(at_node())), nt = __popcll(__ballot(at_tris()));
+      if (nt == 0 || nt < nn || nt < nl - nn - nt || (more && nl <= 4 * (16 - kSceneRefill))) break;
+      if (at_tris()) {
+        // ---- triangle step: four triangles of the leaf ----
+        if (s + q4 < e) {
+          const Tri tr = load_tri(tris, s + q4);
+          const uint32_t mask = A.side_mask ? A.side_mask : tr.mask();
+          float t = 0.0f, et = 0.0f;
+          const RayBand band = ray_band<false>(z, z, fabsf(d.x) + fabsf(d.y) + fabsf(d.z));
+          const float dlen = window ? sqrtf(dot(d, d)) : 1.0f;
+          const int res = hit_fast<false>(o, d, dlen, band, tr, mask, window ? near_t : 0.0f, window ? far_t : kInf, t, et);
+          float lb = t - et;
+          if (res == kUnsure) lb = unsure_from(rb, tr);
+          if (res != kMiss && !(lb > U)) {
+            if (res == kHit) U = fminf(U, t + et);
+            if (cl.n < kCand || cl.compact(U))
+              cl.put(cl.n++, s + q4, lb);
+            else
+              give_up = true;  // more live candidates than the list holds: the one-lane kernel settles them
+          }
+        }
+        give_up = quad_any(give_up);
+        U = fminf(U, quad_xor1(U));
+        U = fminf(U, quad_xor2(U));
+        s += 4;
+        if (give_up)
+          live = false;
+        else
+          settle();
+      }
+    }
+    const bool at_switch = live && !at_node() && !at_tris();
+    const int ns = __popcll(__ballot(at_switch));
+    if (ns >= __popcll(__ballot(at_node())) && ns >= __popcll(__ballot(at_tris())) && at_switch) {
+      // ---- switch: leave the instance (or go on to its next root), enter the next ----
+      if (inst != kNoHit && ++root < mesh->n_roots) {
+        ref = mesh->roots4[root];
+        settle();
+      } else {
+        if (inst != kNoHit) {
+          if (cl.n) cl.compact(U);
+          float lo = kInf;  // the least lower bound of the live candidates (NaN: none known)
+          for (int i = 0; i < cl.n; i++) {
+            const float lb = __uint_as_float(cl.get(i).y);
+            lo = lb == lb ? fminf(lo, lb) : -kInf;
+          }
+          lo = fminf(lo, quad_xor1(lo));
+          lo = fminf(lo, quad_xor2(lo));
+          if (lo < kInf) {  // the quad has live candidates
+            const float slack = span.off + span.grow * U;
+            const float hi_w = U * span.along + slack, lo_w = lo * span.along - slack;
+            if (!(lo_w > best_hi)) {
+              if (hi_w < best_lo) {
+                held = 0;
+                best_lo = lo_w;
+                best_hi = hi_w;
+              } else {
+                // a NaN end stays: nothing is certain then
+                best_lo = lo_w < best_lo || lo_w != lo_w ? lo_w : best_lo;
+                best_hi = hi_w < best_hi || hi_w != hi_w ? hi_w : best_hi;
+              }
+              for (int i = 0; i < cl.n; i++) {
+                if (held < kContend)
+                  contend[held++ * kBlock + lane] = make_uint2(cl.get(i).x, inst);
+                else
+                  give_up = true;
+              }
+              give_up = quad_any(give_up);
+              if (give_up) live = false;
+            }
+          }
+          cl.n = 0;
+          to_top();
+          ref = kDone;
+          if (live) settle();
+        }
+        if (live && inst == kNoHit && ref == kDone && s < e) {
+          const uint4* rec = A.slots + static_cast<uint64_t>(kSceneSlotRows) * s;
+          const uint4 r0 = rec[0], r1 = rec[1], r6 = rec[6];
+          const float4 r7 = reinterpret_cast<const float4*>(rec)[7];
+          const f3 ow = load3(A.origins, ray), dw = load3(A.directions, ray);
+          inst = r0.x;
+          ts = s + 1;
+          te = e;
+          const float4* inv = reinterpret_cast<const float4*>(rec + 2);
+          const float4 i0 = inv[0], i1 = inv[1], i2 = inv[2], i3 = inv[3];
+          const float ie[16] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w,
+                                i2.x, i2.y, i2.z, i2.w, i3.x, i3.y, i3.z, i3.w};
+          mesh = A.meshes + r0.y;
+          nodes = reinterpret_cast<const float4*>((static_cast<uint64_t>(r1.y) << 32) | r1.x);
+          tris = reinterpret_cast<const float4*>((static_cast<uint64_t>(r6.y) << 32) | r6.x);
+          const float coord_max = *reinterpret_cast<const float*>((static_cast<uint64_t>(r1.w) << 32) | r1.z);
+          if (r6.z) {  // an affine inverse: apply_matrix4's divisor is 1 / 1
+            MBVH_NO_CONTRACT
+            o = mk(ie[0] * ow.x + ie[4] * ow.y + ie[8] * ow.z + ie[12], ie[1] * ow.x + ie[5] * ow.y + ie[9] * ow.z + ie[13],
+                   ie[2] * ow.x + ie[6] * ow.y + ie[10] * ow.z + ie[14]);
+          } else {
+            o = apply_matrix4(ie, ow);
+          }
+          d = transform_direction(ie, dw);
+          if (r6.w) {  // the inverse is W's: W3 d = dw / |inverse dw| and W o = ow, up to their roundings
+            const f3 di = mk(ie[0] * dw.x + ie[4] * dw.y + ie[8] * dw.z, ie[1] * dw.x + ie[5] * dw.y + ie[9] * dw.z,
+                             ie[2] * dw.x + ie[6] * dw.y + ie[10] * dw.z);
+            constexpr float kRound = 1.0f / 524288.0f;  // 2^-19
+            const float wo = fabsf(ow.x) + fabsf(ow.y) + fabsf(ow.z);
+            span.along = wlen * __builtin_amdgcn_rsqf(dot(di, di));
+            span.off = (r7.y + kRound) * wo + r7.z + kRound * (r7.x * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z)));
+            span.grow = 2.0f * kRound * r7.x + r7.y * span.along;
+          } else {
+            span = world_span(A.world + 16ull * inst, ow, o, d);
+          }
+          near_t = 0.0f;
+          far_t = kInf;
+          if (window || r0.w) {  // r0.w: a column of matrixWorld without a finite positive length
+            const float sc = instance_scale(A.world + 16ull * inst, d);
+            near_t = A.near_dist / sc;
+            far_t = A.far_dist / sc;
+          }
+          if (!scene_box4(o, d, coord_max, rb)) {
+            give_up = true;
+            live = false;
+          } else {
+            U = kInf;
+            if (best_hi < kInf) {  // no hit farther than the contenders' least upper end can win
+              U = (best_hi + span.off) * rcp_approx(span.along - 2.0f * span.grow) * (1.0f + 1.0f / 65536.0f);
+              if (!(span.along > 2.0f * span.grow) || !(U < kInf)) U = kInf;
+            }
+            base = st.sp;
+            root = 0;
+            s = e = 0;
+            ref = r0.z;
+            settle();
+          }
+        }
+      }
+    }
+  }
+}
+
+// The contenders of the rays settled, one lane per ray.
+__global__ __launch_bounds__(kBlock) void k_scene_ray_resolve(SceneArgs A) {
+  const uint64_t ray = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (ray >= A.n) return;
+  const uint2* c = A.contenders + kSceneRow * ray;
+  const uint2 c0 = c[0];
+  if (c0.x == kOverflow) return;  // left to the one-lane kernel
+  uint32_t count = 0;
+  if (c0.x == kPooled) {
+    count = c[1].x;
+    c = A.contender_pool + c0.y;
+  } else {
+    while (count < kSceneRow && c[count].x != kNoHit) count++;
+  }
+  const f3 ow = load3(A.origins, ray), dw = load3(A.directions, ray), z = mk(0.0f, 0.0f, 0.0f);
+  FirstHit best = no_hit();
+  uint32_t best_inst = kNoHit;
+  for (uint32_t done = 0; done < count; done++) {
+    const uint32_t inst = c[done].y;
+    bool first = true;  // each instance once, at its first contender
+    for (uint32_t i = 0; i < done; i++) first = first && c[i].y != inst;
+    if (!first) continue;
+    const MeshView M = A.meshes[A.instance_geometry[inst]];
+    const float* inv = A.inverse + 16ull * inst;
+    const f3 o = apply_matrix4(inv, ow), d = transform_direction(inv, dw);
+    const float sc = instance_scale(A.world + 16ull * inst, d);
+    const Window win = window_of(A.near_dist / sc, 0.0f, A.far_dist / sc, 0.0f);
+    uint32_t w = kNoHit;
+    ff best_t = {kInf, 0.0f};
+    for (uint32_t i = done; i < count; i++) {
+      if (c[i].y != inst) continue;
+      const uint32_t slot = c[i].x;
+      const Tri tr = load_tri(M.tris, slot);
+      ff t;
+      if (!hit_exact<false>(o, d, z, z, tr.a(), tr.b(), tr.c(), A.side_mask ? A.side_mask : tr.mask(), win, t)) continue;
+      bool take = w == kNoHit;
+      if (!take)
+        take = near_tie(t, best_t) ? slot != w && ray_first_of(tie_tree(M), d.x, d.y, d.z, slot, w)
+                                   : ff_sign(ff_sub(t, best_t)) < 0;
+      if (take) {
+        w = slot;
+        best_t = t;
+      }
+    }
+    if (w == kNoHit) continue;
+    FirstHit h = finish_hit<false>(M.tris, w, o, d, z, z);
+    h.p = apply_matrix4(A.world + 16ull * inst, h.p);
+    h.dist = world_distance(h.p, ow);
+    if (h.dist < best.dist || (h.dist == best.dist && inst < best_inst)) {
+      best = h;
+      best_inst = inst;
+    }
+  }
+  A.out_face[ray] = best.face;
+  if (A.out_instance) A.out_instance[ray] = best_inst;
+  if (A.out_dist) A.out_dist[ray] = best.dist;
+  if (A.out_point) {
+    A.out_point[3 * ray + 0] = best.p.x;
+    A.out_point[3 * ray + 1] = best.p.y;
+    A.out_point[3 * ray + 2] = best.p.z;
+  }
+  if (A.out_bary) {
+    A.out_bary[3 * ray + 0] = best.bary.x;
+    A.out_bary[3 * ray + 1] = best.bary.y;
+    A.out_bary[3 * ray + 2] = best.bary.z;
   }
 }
 
@@ -3779,6 +4308,20 @@ hipError_t launch_batch_raycast_first(const BatchArgs& a, uint32_t stack_lds, ui
     hipLaunchKernelGGL((k_batch_raycast_first<16, true>), dim3(blocks), dim3(kBlock), 0, s, a);
   else
     hipLaunchKernelGGL((k_batch_raycast_first<16, false>), dim3(blocks), dim3(kBlock), 0, s, a);
+  return hipGetLastError();
+}
+
+__global__ void k_scene_ray_reset(uint32_t* queue, uint32_t* count, uint32_t* pool_count) {
+  if (threadIdx.x < kWalkQueues) queue[32 * threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *count = *pool_count = 0u;
+}
+
+hipError_t launch_scene_raycast_first4(const SceneArgs& a, uint64_t quads, hipStream_t s) {
+  if (a.n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_scene_ray_reset, dim3(1), dim3(64), 0, s, a.queue, a.heavy_count,
+                     a.contender_pool_count);
+  hipLaunchKernelGGL(k_scene_raycast_first4, dim3(static_cast<uint32_t>(quads / (kBlock / 4))), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_scene_ray_resolve, dim3(static_cast<uint32_t>((a.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a);
   return hipGetLastError();
 }
 
