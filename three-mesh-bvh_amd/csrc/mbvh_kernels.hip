@@ -2442,10 +2442,33 @@ __global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
 // instructions, the rest being copies of the walk's state).
 // ------------------------------------------------------------------------------------------
 constexpr int kSceneRefill = 3;           // 2 and 6 measured 1 and 2% slower
-constexpr int kSceneLds = 32;             // stack entries per quad in LDS
+constexpr int kSceneLds = 24;             // stack entries per quad in LDS
+constexpr int kSceneCand = 8;             // candidates per lane within an instance
+// Cands over an array of the kernel's own.
+struct SceneCands {
+  uint2* list;
+  uint32_t lane;
+  int n;
+  __device__ __forceinline__ void put(int i, uint32_t slot, float lb) {
+    lds_store(list, i * kBlock + lane, make_uint2(slot, __float_as_uint(lb)));
+  }
+  __device__ __forceinline__ uint2 get(int i) const { return lds_load(list, i * kBlock + lane); }
+  __device__ __forceinline__ bool compact(float U) {
+    int m = 0;
+    for (int i = 0; i < n; i++) {
+      const uint2 e = get(i);
+      if (!(__uint_as_float(e.y) > U)) {
+        if (m != i) put(m, e.x, __uint_as_float(e.y));
+        m++;
+      }
+    }
+    n = m;
+    return n < kSceneCand;
+  }
+};
 constexpr uint32_t kSceneBatch = 64;
 constexpr uint32_t kPooled = 0xFFFFFFFDu;  // a row's first word: its contenders are in the pool
-constexpr int kContend = 4;               // contenders per lane
+constexpr uint32_t kContend = 16;         // contenders a quad holds
 
 // ray_box4 for the scene's quads: the reciprocals by the hardware's 1-ulp instruction. That is u more
 // relative error than a division on both plane products, 6 u S of the widening's 8 u S. False: a zero
@@ -2522,7 +2545,8 @@ struct SceneStack {
 
 __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A) {
   __shared__ uint2 qstack[kSceneLds * (kBlock / 4)];
-  __shared__ uint2 contend[kContend * kBlock];  // (slot, instance)
+  __shared__ uint2 clist[kSceneCand * kBlock];
+  __shared__ uint2 contend[kContend * (kBlock / 4)];  // (slot, instance)
   __shared__ float4 wbox[2 * (kBlock / 4)];
   __shared__ float wbox_hz[kBlock / 4];
   const uint32_t lane = threadIdx.x, wl = lane & 63u, q4 = lane & 3u, qid = lane >> 2;
@@ -2551,10 +2575,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
   f3 o = z, d = z;
   RayBox4 rb = {};
   float U = kInf, near_t = 0.0f, far_t = kInf;
-  Cands cl;
-  cl.lane = lane;
-  cl.n = 0;
-  int held = 0;                               // this lane's contenders
+  SceneCands cl = {clist, lane, 0};
+  uint32_t held = 0;                          // the quad's contenders
   float best_lo = kInf, best_hi = kInf;       // the contenders' world distances
 
   float wlen = 1.0f;                          // length of the world direction
@@ -2610,20 +2632,17 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
     if (idle == 16 || (idle >= kSceneRefill && (tried < kWalkQueues || cur < end))) {
       // ---- the finished rays' contenders, then new rays ----
       if (!live && ray != kNoHit) {
-        const uint32_t h = static_cast<uint32_t>(held);
-        const uint32_t h0 = quad_bcast<0>(h), h1 = quad_bcast<1>(h), h2 = quad_bcast<2>(h), h3 = quad_bcast<3>(h);
-        const uint32_t total = h0 + h1 + h2 + h3;
         uint2* const row = A.contenders + static_cast<uint64_t>(kSceneRow) * ray;
         uint2* to = row;
-        if (!give_up && total > kSceneRow) {  // a row of the pool, named in the ray's own
+        if (!give_up && held > kSceneRow) {  // a row of the pool, named in the ray's own
           uint32_t at = 0;
-          if (q4 == 0) at = atomicAdd(A.contender_pool_count, total);
+          if (q4 == 0) at = atomicAdd(A.contender_pool_count, held);
           at = quad_bcast<0>(at);
-          give_up = at > A.contender_pool_cap || A.contender_pool_cap - at < total;
+          give_up = at > A.contender_pool_cap || A.contender_pool_cap - at < held;
           to = A.contender_pool + at;
           if (q4 == 0 && !give_up) {
             row[0] = make_uint2(kPooled, at);
-            row[1] = make_uint2(total, 0u);
+            row[1] = make_uint2(held, 0u);
           }
         }
         if (give_up) {
@@ -2632,9 +2651,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
             row[0] = make_uint2(kOverflow, 0u);  // not for the resolution
           }
         } else {
-          uint32_t at = q4 == 0 ? 0u : (q4 == 1 ? h0 : (q4 == 2 ? h0 + h1 : h0 + h1 + h2));
-          for (uint32_t i = 0; i < h; i++) to[at++] = contend[i * kBlock + lane];
-          if (q4 == 3 && total < kSceneRow) row[total] = make_uint2(kNoHit, 0u);
+          for (uint32_t i = q4; i < held; i += 4) to[i] = contend[i * (kBlock / 4) + qid];
+          if (q4 == 0 && held < kSceneRow) row[held] = make_uint2(kNoHit, 0u);
         }
         ray = kNoHit;
       }
@@ -2658,7 +2676,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
       if (!live && rank < take) {
         ray = cur + rank;
         best_lo = best_hi = kInf;
-        held = cl.n = 0;
+        held = 0;
+        cl.n = 0;
         ts = te = 0;
         st.sp = 0;
         const f3 ow = load3(A.origins, ray), dw = load3(A.directions, ray);
@@ -2719,7 +2738,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
           if (res == kUnsure) lb = unsure_from(rb, tr);
           if (res != kMiss && !(lb > U)) {
             if (res == kHit) U = fminf(U, t + et);
-            if (cl.n < kCand || cl.compact(U))
+            if (cl.n < kSceneCand || cl.compact(U))
               cl.put(cl.n++, s + q4, lb);
             else
               give_up = true;  // more live candidates than the list holds: the one-lane kernel settles them
@@ -2765,14 +2784,18 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
                 best_lo = lo_w < best_lo || lo_w != lo_w ? lo_w : best_lo;
                 best_hi = hi_w < best_hi || hi_w != hi_w ? hi_w : best_hi;
               }
-              for (int i = 0; i < cl.n; i++) {
-                if (held < kContend)
-                  contend[held++ * kBlock + lane] = make_uint2(cl.get(i).x, inst);
-                else
-                  give_up = true;
+              const uint32_t h = static_cast<uint32_t>(cl.n);
+              const uint32_t h0 = quad_bcast<0>(h), h1 = quad_bcast<1>(h), h2 = quad_bcast<2>(h), h3 = quad_bcast<3>(h);
+              const uint32_t total = h0 + h1 + h2 + h3;
+              if (held + total > kContend) {
+                give_up = true;
+                live = false;
+              } else {
+                const uint32_t to = held + (q4 == 0 ? 0u : (q4 == 1 ? h0 : (q4 == 2 ? h0 + h1 : h0 + h1 + h2)));
+                for (uint32_t i = 0; i < h; i++)
+                  contend[(to + i) * (kBlock / 4) + qid] = make_uint2(cl.get(static_cast<int>(i)).x, inst);
+                held += total;
               }
-              give_up = quad_any(give_up);
-              if (give_up) live = false;
             }
           }
           cl.n = 0;
