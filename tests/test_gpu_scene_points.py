@@ -1,0 +1,109 @@
+"""The scene closest point's FP32 walk (instances placed by similarities) where its bounds and lists could
+go wrong: ties between many triangles and instances, points its lists cannot hold, far, tiny and
+non-finite queries, large and small scales. The answer is the one-lane kernel's, which measures in
+double as it walks, bit for bit."""
+import numpy as np
+import pytest
+
+import mbvh_amd as M
+from mbvh_amd import geometry as G
+from helpers import build_mesh
+
+pytestmark = pytest.mark.gpu
+
+GEOMS = [lambda: G.sphere(1.0, 60, 40), lambda: G.torus_knot(0.8, 0.25, 90, 9, 2, 3), lambda: G.sphere(0.7, 3, 2)]
+
+
+@pytest.fixture(scope="module")
+def setup():
+    ctx = M.Context(0)
+    built = [build_mesh(f()) for f in GEOMS]
+    meshes = [ctx.upload(t, g.positions, idx) for g, idx, t in built]
+    yield ctx, meshes
+    for m in meshes:
+        m.free()
+    ctx.close()
+
+
+def matrices(count, rng, scale=(0.5, 2.0), span=6.0, stretch=1.0):
+    q = rng.normal(size=(count, 4))
+    x, y, z, w = (q / np.linalg.norm(q, axis=1, keepdims=True)).T
+    r = np.stack([1 - 2 * (y * y + z * z), 2 * (x * y - z * w), 2 * (x * z + y * w),
+                  2 * (x * y + z * w), 1 - 2 * (x * x + z * z), 2 * (y * z - x * w),
+                  2 * (x * z - y * w), 2 * (y * z + x * w), 1 - 2 * (x * x + y * y)], axis=1).reshape(-1, 3, 3)
+    m = np.zeros((count, 4, 4))
+    m[:, :3, :3] = r * rng.uniform(*scale, size=(count, 1, 1)) * np.array([1.0, 1.0, stretch])
+    m[:, :3, 3] = rng.uniform(-span, span, size=(count, 3))
+    m[:, 3, 3] = 1
+    return m
+
+
+def check(setup, m, which, points):
+    ctx, meshes = setup
+    world = np.ascontiguousarray(m.transpose(0, 2, 1).reshape(-1, 16), dtype=np.float32)
+    inverse = np.linalg.inv(world.reshape(-1, 4, 4).astype(np.float64)).reshape(-1, 16).astype(np.float32)
+    sc = ctx.scene(meshes, world, inverse, np.asarray(which, dtype=np.uint32))
+    points = np.ascontiguousarray(points, dtype=np.float32)
+    got = sc.closest_point(points)
+    ctx.set_point_lanes(1)
+    ref = sc.closest_point(points)
+    ctx.set_point_lanes(0)
+    sc.free()
+    for k in ref:
+        np.testing.assert_array_equal(got[k].view(np.uint32), ref[k].view(np.uint32), err_msg=k)
+    return ref
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 65, 3001])
+@pytest.mark.parametrize("count", [1, 2, 40])
+def test_counts(setup, n, count):
+    rng = np.random.default_rng(n + count)
+    ref = check(setup, matrices(count, rng), rng.integers(0, 3, count), rng.uniform(-7, 7, size=(n, 3)))
+    assert np.all(ref["face"] != M.NO_HIT)
+
+
+@pytest.mark.parametrize("copies,n", [(2, 2000), (40, 2000), (40, 20000)])
+def test_coincident_instances(setup, copies, n):
+    """Every triangle ties with its copies: past a row, past a lane's list, more such points than a wave each."""
+    rng = np.random.default_rng(copies)
+    m = np.repeat(matrices(2, rng), copies, axis=0)
+    ref = check(setup, m, np.repeat([0, 1], copies), rng.uniform(-5, 5, size=(n, 3)))
+    assert np.all(ref["instance"] % copies == 0)
+
+
+@pytest.mark.parametrize("spread", [0.0, 1e-4])
+def test_long_walks(setup, spread):
+    """Points at the centres of spheres, on their poles and axes, and on vertices."""
+    rng = np.random.default_rng(3)
+    m = matrices(6, rng)
+    local = np.concatenate([np.zeros((60, 3)), np.tile([[0, 1, 0], [0, -1, 0], [0, 3, 0], [0, 0.2, 0]], (60, 1)),
+                            G.sphere(1.0, 60, 40).positions.reshape(-1, 3)[:200]]) + spread * rng.normal(size=(500, 3))
+    at = rng.integers(0, 6, 500)
+    check(setup, m, [0] * 6, np.einsum("nij,nj->ni", m[at][:, :3, :3], local) + m[at][:, :3, 3])
+
+
+@pytest.mark.parametrize("size", [1e3, 1e6, 1e15, 3e19, 1e-10])
+def test_far_and_tiny(setup, size):
+    rng = np.random.default_rng(5)
+    check(setup, matrices(5, rng), [0, 1, 2, 0, 1], size * rng.normal(size=(300, 3)))
+
+
+@pytest.mark.parametrize("scale,span", [((1e-5, 1e-4), 1e-3), ((1e4, 1e5), 1e5), ((1e-3, 1e3), 50.0), ((1.0, 1.0), 1e4)])
+def test_scales(setup, scale, span):
+    rng = np.random.default_rng(6)
+    check(setup, matrices(12, rng, scale, span), rng.integers(0, 3, 12), span * rng.uniform(-1.2, 1.2, size=(2000, 3)))
+
+
+@pytest.mark.parametrize("stretch", [1.0 + 1e-7, 1.0 + 1e-5, 1.0 + 1e-4, 1.5, -1.0])
+def test_stretched(setup, stretch):
+    """Either side of the similarity rule, and mirrored."""
+    rng = np.random.default_rng(7)
+    check(setup, matrices(12, rng, stretch=stretch), rng.integers(0, 3, 12), rng.uniform(-7, 7, size=(2000, 3)))
+
+
+def test_not_finite(setup):
+    rng = np.random.default_rng(8)
+    p = rng.uniform(-7, 7, size=(64, 3))
+    p[0::8, 0], p[1::8, 1], p[2::8] = np.nan, np.inf, -np.inf
+    ref = check(setup, matrices(3, rng), [0, 1, 2], p)
+    assert np.all(ref["face"][0::8] == M.NO_HIT) and np.all(ref["face"][3::8] != M.NO_HIT)

@@ -266,9 +266,10 @@ struct BatchArgs {
 };
 
 constexpr uint32_t kSceneRow = 4;       // contenders of a ray before it takes a row of the pool
-constexpr uint32_t kScenePool = 1u << 20;  // pool entries per launch; when they are gone, the one-lane kernel
+constexpr uint32_t kScenePool = 1u << 22;  // pool entries per launch; when they are gone, the one-lane kernel
 constexpr uint32_t kSceneSlotRows = 8;  // uint4 per top-level slot
 // Scene: closest first hit over instances, one launch (TLAS over the instances' world boxes).
+constexpr uint32_t kScenePointRows = 10;
 struct SceneArgs {
   const MeshView* meshes;
   uint32_t n_meshes;
@@ -285,6 +286,11 @@ struct SceneArgs {
   // address, whether that inverse is affine, whether it is matrixWorld's to 2^-20), the magnitudes of their
   // products (sum of |W3|; 2^-18 times the largest row sum of |W3| |R3|; 2^-18 times that of the translations)
   const uint4* slots;
+  // closest point, four lanes: per slot of that tree, kScenePointRows rows: (instance, mesh, the mesh's
+  // first 4-wide root, 0), (nodes4, frames: device addresses), (matrixWorld's translation, 0), (s_lo,
+  // s_hi, s_hi / s_lo, 1 / s_lo: bounds of its singular values), the inverse of its 3x3 part (nine doubles, row
+  // by row, and one of padding); NULL: some instance is no similarity
+  const uint4* point_slots;
   uint2* contenders;               // kSceneRow (triangle slot, instance) per ray, ended by kNoHit when fewer
   uint2* contender_pool;           // rows of the rays with more
   uint32_t* contender_pool_count;
@@ -317,6 +323,13 @@ struct SceneArgs {
   uint32_t* heavy;
   uint32_t* heavy_count;
   uint32_t heavy_budget;
+  // closest point: the points (positions in the visit order) the FP32 walk left for the size of their
+  // lists, then those the wave-per-point kernel left, with both counts, and the FP64 walk's work queue;
+  // NULL: that walk takes every point
+  uint32_t* rest;
+  uint32_t* rest_count;
+  uint32_t* more_count;
+  uint32_t* rest_queue;
 };
 // One lane per ray, over a.heavy (*a.heavy_count rays) or, when it is NULL, every ray.
 hipError_t launch_scene_raycast_first(const SceneArgs& a, uint64_t threads, hipStream_t s);
@@ -332,6 +345,11 @@ hipError_t launch_scene_closest_point4(const SceneArgs& a, uint64_t threads, hip
 // LDS frontier of kWideFrontier entries; `waves` persistent waves. The instance trees' 4-wide depth
 // must fit that frontier: 64 * (max_stack4 - 1) + 256 <= kWideFrontier.
 constexpr uint32_t kWideFrontier = 4096;
+// The same where every instance is placed by a similarity (a.point_slots): the walk in FP32 with four
+// lanes per point, then a wave for each long one (a.heavy, a.n entries), and the resolution of their
+// candidates; what is left is listed in a.rest (2 a.n entries, a.n < 2^32) for launch_scene_closest_point4
+// (many points) and launch_scene_closest_point_wide (those even a wave's lists cannot hold).
+hipError_t launch_scene_point_walk4(const SceneArgs& a, uint64_t quads, hipStream_t s);
 hipError_t launch_scene_closest_point_wide(const SceneArgs& a, uint32_t waves, hipStream_t s);
 
 // ---- intersectsBox ----------------------------------------------------------------------------------

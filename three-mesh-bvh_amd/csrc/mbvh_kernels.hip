@@ -2467,6 +2467,11 @@ struct SceneCands {
   }
 };
 constexpr uint32_t kSceneBatch = 64;
+// Points the FP32 walk leaves for the size of their lists get a wave each up to this many, four lanes in
+// FP64 beyond: 40 coincident spheres of 40,000 triangles, 30,000 points 74 ms against 100, 262,144
+// points 560 ms against 467.
+constexpr uint32_t kSceneRestWide = 65536;
+constexpr uint64_t kScenePointWaves = 4096;
 constexpr uint32_t kPooled = 0xFFFFFFFDu;  // a row's first word: its contenders are in the pool
 constexpr uint32_t kContend = 16;         // contenders a quad holds
 
@@ -3969,6 +3974,8 @@ __device__ __forceinline__ bool scene_point_instance4(const MeshView& M, const f
 
 __device__ __forceinline__ void scene_point_out(const SceneArgs& A, uint64_t i, bool overflow, ScenePick b, D3 p);
 
+// kRest: the points the FP32 walk left (A.rest), where they are many; otherwise every point.
+template <bool kRest>
 __global__ __launch_bounds__(kBlock, 4) void k_scene_closest_point4(SceneArgs A) {
   __shared__ uint2 qstack[kQuadLds * (kBlock / 4)];
   const uint32_t lane = threadIdx.x, q4 = lane & 3u, wq = (lane & 63u) >> 2, qid = lane >> 2;
@@ -3979,20 +3986,23 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_closest_point4(SceneArgs A)
   st.gquad = static_cast<uint64_t>(blockIdx.x) * (kBlock / 4) + qid;
   st.qid = qid;
   st.capacity = kQuadLds + static_cast<int>(A.stack.ovf_entries);
+  const uint64_t n = kRest ? static_cast<uint64_t>(*A.rest_count) : A.n;
+  if (kRest && n <= kSceneRestWide) return;
   while (true) {
     uint32_t tile = 0;
     if ((lane & 63u) == 0) tile = atomicAdd(A.queue, 1u);
     tile = __shfl(tile, 0, 64);
-    if (static_cast<uint64_t>(tile) * 16 >= A.n) break;  // every wave reaches this exit
+    if (static_cast<uint64_t>(tile) * 16 >= n) break;  // every wave reaches this exit
     const uint64_t visit = static_cast<uint64_t>(tile) * 16 + wq;
-    if (visit >= A.n) continue;
-    const uint64_t i = A.order ? A.order[visit] : visit;
+    if (visit >= n) continue;
+    const uint64_t v = kRest ? A.rest[visit] : visit;
+    const uint64_t i = A.order ? A.order[v] : v;
     const float px = A.origins[3 * i], py = A.origins[3 * i + 1], pz = A.origins[3 * i + 2];
     ScenePick b = {__builtin_huge_val(), kNoHit, kNoHit, kNoHit};
     float ubw = kInf;  // an upper bound of the least world squared distance, from FP32 distances
     bool overflow = false;
     uint32_t steps = 0;
-    const uint32_t budget = A.heavy ? A.heavy_budget : 0xFFFFFFFFu;
+    const uint32_t budget = !kRest && A.heavy ? A.heavy_budget : 0xFFFFFFFFu;
     st.sp = 0;
     uint32_t node = 0;  // the root is always entered (an empty scene's is an empty leaf)
     while (true) {
@@ -4040,6 +4050,453 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_closest_point4(SceneArgs A)
 }
 
 // ------------------------------------------------------------------------------------------
+// Scene closest point where every instance is placed by a similarity (rotation, reflection and one
+// scale, to 2^-13; the scene says so): four lanes per point over the 4-wide top level and the
+// instances' trees, both walked by one loop in FP32, the FP64 distances left to k_scene_point_resolve.
+//
+// In an instance the point is l = R (p - t), R the inverse of W's 3x3 part, computed in double and
+// rounded: within delta = 2 u |l| of the exact local point (its norm's bound; kept in double because a
+// looser delta lists more triangles: six instead of two per point in FP32). World distances are
+// between s_lo and s_hi times local ones (the least and largest singular value of W's 3x3 part), so a
+// triangle whose local distance is at most h bounds the best world distance by s_hi (h + delta), and
+// anything farther than (s_hi (h + delta)) / s_lo + delta from l in the instance can neither win nor
+// tie. Triangles are measured by their frames. The record of an instance holds those constants,
+// rounded outward. 1e-30 on the bounds covers underflow.
+//
+// A lane lists the triangles that may still win or tie with the instance and a lower bound of their world
+// distance, one of them in registers (the packets' rule). A point past the step budget goes to a wave of
+// its own (A.heavy, the kernel after this), one with more candidates than the lists hold to A.rest.
+//
+// What bounds it: latency and the vector-memory unit, at five waves per SIMD (512 instances of up to
+// 50,000 triangles, 2^20 points in Morton order: 7 top-level and 23 tree nodes, 113 triangles in 16
+// leaves per point, a wave's longest point 1.8 times that; 1.7 of 3.6 ms is vector issue). The kernel it
+// replaces there measured in FP64 as it walked the binary top level and each instance in a nest of
+// loops, with 128 registers and spills: 8.4 ms. The budget keeps the longest points from
+// outlasting the launch: 4.4 ms at 256 steps, 3.5 at 100, 3.2 at 64 (where the wave kernel takes 1.4 ms).
+// ------------------------------------------------------------------------------------------
+constexpr int kPointCand = 4;       // listed candidates per lane, besides the one in registers
+constexpr int kPointWideCand = 12;  // the same where a point has a wave
+constexpr float kTiny = 1e-30f;
+
+__device__ __forceinline__ float wave_min_f(float v) {
+  for (int m = 1; m < 64; m <<= 1) v = fminf(v, __shfl_xor(v, m, 64));
+  return v;
+}
+
+// Exclusive prefix sum of c over the wave; *total receives the sum.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t c, uint32_t lane, uint32_t* total) {
+  uint32_t x = c;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, 64);
+    if (lane >= static_cast<uint32_t>(d)) x += y;
+  }
+  *total = __shfl(x, 63, 64);
+  return x - c;
+}
+
+// A lane's bounds and candidates. U: upper bound of the point's best squared world distance. T: the
+// threshold of squared distances from q in the frame walked.
+template <int kCap>
+struct ScenePointLane {
+  uint2* list;      // kCap entries for each of the block's lanes: (slot, lower bound)
+  uint32_t* insts;  // their instances
+  uint32_t lane, stride;
+  float U, T;
+  uint32_t near_slot, near_inst;
+  float near_lb;
+  int n;
+  bool full;        // a candidate found no place
+  // the instance walked
+  f3 q;
+  float s_lo, s_hi, ratio, delta;
+
+  __device__ __forceinline__ void start() {
+    U = T = near_lb = kInf;
+    near_slot = near_inst = kNoHit;
+    n = 0;
+    full = false;
+  }
+  __device__ __forceinline__ void compact() {
+    int m = 0;
+    for (int k = 0; k < n; k++) {
+      const uint2 e = lds_load(list, k * stride + lane);
+      if (__uint_as_float(e.y) > U) continue;
+      if (m != k) {
+        lds_store(list, m * stride + lane, e);
+        insts[m * stride + lane] = insts[k * stride + lane];
+      }
+      m++;
+    }
+    n = m;
+  }
+  // Enters the instance of a record: its constants, the point in its frame, T from U.
+  __device__ __forceinline__ void enter(const uint4* rec, f3 p) {
+    const float4* const f = reinterpret_cast<const float4*>(rec);
+    const double2* const m = reinterpret_cast<const double2*>(rec + 4);
+    const float4 t = f[2], k = f[3];
+    const double2 m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3], m4 = m[4];
+    const double x = static_cast<double>(p.x) - t.x, y = static_cast<double>(p.y) - t.y, z = static_cast<double>(p.z) - t.z;
+    q = mk(static_cast<float>(m0.x * x + m0.y * y + m1.x * z), static_cast<float>(m1.y * x + m2.x * y + m2.y * z),
+           static_cast<float>(m3.x * x + m3.y * y + m4.x * z));
+    s_lo = k.x;
+    s_hi = k.y;
+    ratio = k.z;
+    delta = 2.0f * kU * __builtin_amdgcn_sqrtf(dot(q, q)) + kTiny;
+    const float t1 = fmaf(sqrt_up(U), k.w, fmaf(delta, ratio, delta));
+    T = t1 * t1 * (1.0f + 16.0f * kU) + kTiny;
+  }
+  // Measures triangle `slot` of instance `inst`.
+  __device__ __forceinline__ void test(const float4* frames, uint32_t slot, uint32_t inst) {
+    const float4* const fr = frames + static_cast<uint64_t>(kFrameRows) * slot;
+    const float4 f0 = fr[0];
+    const float d2 = frame_dist2(q, f0, fr[1], fr[2], fr[3], fr[4]);
+    const float e2 = frame_error<false>(d2, f0.w, 0.0f);
+    const float lo = d2 - e2;  // NaN: the triangle is left to the exact step
+    if (lo > T) return;
+    const float lb1 = fmaxf(__builtin_amdgcn_sqrtf(lo) * (1.0f - 4.0f * kU) * s_lo - delta * s_hi, 0.0f);
+    const float lb = lb1 * lb1 * (1.0f - 8.0f * kU);
+    bool replace = false;
+    if (!signbit_of(f0.w)) {
+      const float h = sqrt_up(d2 + e2) + delta;
+      const float ub = h * h * (s_hi * s_hi) * (1.0f + 16.0f * kU) + kTiny;
+      const float t1 = fmaf(h, ratio, delta);
+      U = fminf(U, ub);
+      T = fminf(T, t1 * t1 * (1.0f + 16.0f * kU) + kTiny);
+      replace = ub < near_lb;  // the one before can neither win nor tie
+    }
+    if (replace) {
+      near_slot = slot;
+      near_inst = inst;
+      near_lb = lb;
+    } else {
+      if (n == kCap) compact();
+      if (n < kCap) {
+        lds_store(list, n * stride + lane, make_uint2(slot, __float_as_uint(lb)));
+        insts[n * stride + lane] = inst;
+        n++;
+      } else {
+        full = true;
+      }
+    }
+  }
+  // Drops what U excludes; the candidates left.
+  __device__ __forceinline__ uint32_t left() {
+    if (near_lb > U) near_slot = kNoHit;
+    compact();
+    return (near_slot != kNoHit ? 1u : 0u) + static_cast<uint32_t>(n);
+  }
+  __device__ __forceinline__ void write(uint2* to) const {
+    if (near_slot != kNoHit) *to++ = make_uint2(near_slot, near_inst);
+    for (int k = 0; k < n; k++) *to++ = make_uint2(lds_load(list, k * stride + lane).x, insts[k * stride + lane]);
+  }
+};
+
+// Where a point's `total` candidates go: its row or a row of the pool named in it (`first`: the lane that
+// writes for the point; every lane of the point gets `at` from `share`). False: the pool ran out.
+template <typename Share>
+__device__ __forceinline__ bool scene_point_row(const SceneArgs& A, uint64_t v, uint32_t total, bool first, Share share,
+                                                uint2*& to) {
+  uint2* const row = A.contenders + static_cast<uint64_t>(kSceneRow) * v;
+  to = row;
+  if (total > kSceneRow) {
+    uint32_t at = 0;
+    if (first) at = atomicAdd(A.contender_pool_count, total);
+    at = share(at);
+    if (at > A.contender_pool_cap || A.contender_pool_cap - at < total) return false;
+    to = A.contender_pool + at;
+    if (first) {
+      row[0] = make_uint2(kPooled, at);
+      row[1] = make_uint2(total, 0u);
+    }
+  } else if (first && total < kSceneRow) {
+    row[total] = make_uint2(kNoHit, 0u);
+  }
+  return true;
+}
+
+// Whether FP32 squares hold: other points (and those not finite) are left to the FP64 kernels.
+__device__ __forceinline__ bool scene_point_fits(f3 p) { return fabsf(p.x) + fabsf(p.y) + fabsf(p.z) < 1e18f; }
+
+__global__ __launch_bounds__(kBlock, 6) void k_scene_point_walk4(SceneArgs A) {
+  __shared__ uint2 qstack[kSceneLds * (kBlock / 4)];
+  __shared__ uint2 clist[kPointCand * kBlock];
+  __shared__ uint32_t cinst[kPointCand * kBlock];
+  const uint32_t lane = threadIdx.x, wl = lane & 63u, q4 = lane & 3u, qid = lane >> 2;
+  SceneStack st;
+  st.lds = qstack;
+  st.ovf = A.stack.ovf;
+  st.ovf_stride = static_cast<uint64_t>(gridDim.x) * (kBlock / 4);
+  st.gquad = static_cast<uint64_t>(blockIdx.x) * (kBlock / 4) + qid;
+  st.qid = qid;
+  st.capacity = kSceneLds + static_cast<int>(A.stack.ovf_entries);
+  ScenePointLane<kPointCand> L;
+  L.list = clist;
+  L.insts = cinst;
+  L.lane = lane;
+  L.stride = kBlock;
+  const uint32_t n = static_cast<uint32_t>(A.n);
+  const uint32_t batches = (n + kSceneBatch - 1) / kSceneBatch, share = (batches + kWalkQueues - 1) / kWalkQueues;
+  uint32_t cur = 0, end = 0, home = blockIdx.x % kWalkQueues, tried = 0;
+  while (true) {
+    while (cur >= end && tried < kWalkQueues) {
+      uint32_t b = 0;
+      if (wl == 0) b = atomicAdd(A.queue + 32 * home, 1u);
+      b = __builtin_amdgcn_readfirstlane(b);
+      const uint32_t at = home * share + b;
+      if (b < share && at < batches) {
+        cur = at * kSceneBatch;
+        end = min(cur + kSceneBatch, n);
+      } else {
+        home = (home + 1) % kWalkQueues;
+        tried++;
+      }
+    }
+    if (cur >= end) break;  // every wave reaches this exit: the queues only run empty
+    const uint32_t v = cur + (wl >> 2);
+    cur += 16;
+    if (v >= end) continue;
+    const uint64_t i = A.order ? A.order[v] : v;
+    const f3 p = load3(A.origins, i);
+    L.start();
+    uint32_t steps = 0;
+    bool full = false, overflow = !scene_point_fits(p);
+    st.sp = 0;
+    int base = 0;
+    uint32_t inst = kNoHit, ts = 0, te = 0, root = 0, ref = A.tlas4_root;
+    const float4* nodes = A.tlas4;
+    const float4* frames = nullptr;
+    const MeshView* mesh = A.meshes;
+    L.q = p;
+    auto pop = [&]() {
+      while (ref == kDone && st.sp > base) {
+        const uint2 e = st.pop();
+        if (__uint_as_float(e.y) <= L.T) ref = e.x;
+      }
+    };
+    while (!overflow) {
+      while (!(ref & kRefLeaf) && ref != kDone) {
+        const float4 c0 = nodes[8ull * ref + 2 * q4];
+        const float4 c1 = nodes[8ull * ref + 2 * q4 + 1];
+        const uint32_t cref = __float_as_uint(c1.z);
+        const float sc = box_score(L.q, c0.x, c0.y, c0.z, c0.w, c1.x, c1.y) * (1.0f - 4.0f * kU);
+        ref = quad_children(st, lane, (cref != kDone) & (sc <= L.T), sc, cref, overflow);
+        if (overflow) break;
+        pop();
+      }
+      if (overflow) break;
+      if (inst != kNoHit) {
+        while (ref & kRefLeaf) {
+          uint32_t off, cnt;
+          leaf_range(ref, mesh->bigleaf, off, cnt);
+          for (uint32_t s = off + q4; s < off + cnt; s += 4) L.test(frames, s, inst);
+          L.T = fminf(L.T, quad_xor1(L.T));
+          L.T = fminf(L.T, quad_xor2(L.T));
+          L.U = fminf(L.U, quad_xor1(L.U));
+          L.U = fminf(L.U, quad_xor2(L.U));
+          full = quad_any(L.full);
+          ref = kDone;
+          if (full || ++steps > A.heavy_budget) break;
+          pop();
+        }
+        if (full || steps > A.heavy_budget) break;
+        if (ref != kDone) continue;  // a node
+        if (++root < mesh->n_roots) {
+          ref = mesh->roots4[root];
+          continue;
+        }
+        inst = kNoHit;
+        nodes = A.tlas4;
+        L.q = p;
+        L.T = L.U;
+        base = 0;
+      } else if (ref & kRefLeaf) {
+        leaf_range(ref, A.tlas4_bigleaf, ts, te);
+        te += ts;
+        ref = kDone;
+      }
+      // ---- the top level: the next instance of the leaf, or the next entry ----
+      if (ts < te) {
+        const uint4* rec = A.point_slots + static_cast<uint64_t>(kScenePointRows) * ts++;
+        const uint4 r0 = rec[0], r1 = rec[1];
+        inst = r0.x;
+        mesh = A.meshes + r0.y;
+        ref = r0.z;
+        root = 0;
+        nodes = reinterpret_cast<const float4*>((static_cast<uint64_t>(r1.y) << 32) | r1.x);
+        frames = reinterpret_cast<const float4*>((static_cast<uint64_t>(r1.w) << 32) | r1.z);
+        L.enter(rec, p);
+        base = st.sp;
+        continue;
+      }
+      pop();
+      if (ref == kDone) break;
+    }
+    const bool heavy = !full && steps > A.heavy_budget;
+    bool left = full || overflow;
+    if (!heavy && !left) {
+      const uint32_t h = L.left();
+      const uint32_t h0 = quad_bcast<0>(h), h1 = quad_bcast<1>(h), h2 = quad_bcast<2>(h), h3 = quad_bcast<3>(h);
+      uint2* to;
+      left = !scene_point_row(A, v, h0 + h1 + h2 + h3, q4 == 0, [](uint32_t at) { return quad_bcast<0>(at); }, to);
+      if (!left) L.write(to + (q4 == 0 ? 0u : (q4 == 1 ? h0 : (q4 == 2 ? h0 + h1 : h0 + h1 + h2))));
+    }
+    if ((heavy || left) && q4 == 0) {
+      A.contenders[static_cast<uint64_t>(kSceneRow) * v] = make_uint2(kOverflow, 0u);  // not for the resolution yet
+      if (heavy)
+        A.heavy[atomicAdd(A.heavy_count, 1u)] = v;
+      else
+        A.rest[atomicAdd(A.rest_count, 1u)] = v;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The points of A.heavy, and those of A.rest while they are few, a wave each: the same bounds and lists
+// (64 lanes' lists), the nodes of the instance walked on a stack the wave shares. A round takes its top
+// sixteen entries, a quad each: a node's children in reach are pushed, a leaf's triangles measured, and the
+// bounds reduced over the wave. A point that even these lists or the stack cannot hold goes to the end
+// of A.rest (A.more_count of them).
+//
+// What bounds it: the serial rounds of a point (load, reduce, push), eight waves to a compute unit:
+// 0.3 ms for some 5,000 points; one triangle per lane in turn, in FP64, took 0.8 ms for a fifth of them.
+// ------------------------------------------------------------------------------------------
+constexpr uint32_t kPointFrontier = 1024;  // at most 48 entries per level of the tree and 64
+constexpr uint32_t kPointTop = 80;         // the top level's stack: three entries for each of 24 levels
+
+struct PointTopStack {
+  uint2* lds;
+  int capacity, sp;
+  __device__ __forceinline__ void put(int pos, uint32_t ref, uint32_t aux) { lds_store(lds, pos, make_uint2(ref, aux)); }
+};
+
+__global__ __launch_bounds__(64) void k_scene_point_wide(SceneArgs A) {
+  __shared__ uint2 front[kPointFrontier];
+  __shared__ uint2 top[kPointTop];
+  __shared__ uint2 clist[kPointWideCand * 64];
+  __shared__ uint32_t cinst[kPointWideCand * 64];
+  const uint32_t lane = threadIdx.x, q4 = lane & 3u, quad = lane >> 2;
+  ScenePointLane<kPointWideCand> L;
+  L.list = clist;
+  L.insts = cinst;
+  L.lane = lane;
+  L.stride = 64;
+  PointTopStack st = {top, static_cast<int>(kPointTop), 0};
+  const uint32_t nh = *A.heavy_count, rest = *A.rest_count, nr = rest <= kSceneRestWide ? rest : 0u;
+  for (uint32_t h = blockIdx.x; h < nh + nr; h += gridDim.x) {
+    const uint32_t v = h < nh ? A.heavy[h] : A.rest[h - nh];
+    const uint64_t i = A.order ? A.order[v] : v;
+    const f3 p = load3(A.origins, i);
+    L.start();
+    bool overflow = !scene_point_fits(p);
+    st.sp = 0;
+    uint32_t ref = A.tlas4_root;
+    while (ref != kDone && !overflow) {  // the top level, the same in every quad
+      L.q = p;
+      L.T = L.U;
+      if (!(ref & kRefLeaf)) {
+        const float4 c0 = A.tlas4[8ull * ref + 2 * q4], c1 = A.tlas4[8ull * ref + 2 * q4 + 1];
+        const uint32_t cref = __float_as_uint(c1.z);
+        const float sc = box_score(p, c0.x, c0.y, c0.z, c0.w, c1.x, c1.y) * (1.0f - 4.0f * kU);
+        ref = quad_children(st, lane, (cref != kDone) & (sc <= L.T), sc, cref, overflow);
+      } else {
+        uint32_t ts, te;
+        leaf_range(ref, A.tlas4_bigleaf, ts, te);
+        te += ts;
+        ref = kDone;
+        for (; ts < te && !overflow; ts++) {
+          const uint4* rec = A.point_slots + static_cast<uint64_t>(kScenePointRows) * ts;
+          const uint4 r0 = rec[0], r1 = rec[1];
+          const MeshView* const mesh = A.meshes + r0.y;
+          const float4* const nodes = reinterpret_cast<const float4*>((static_cast<uint64_t>(r1.y) << 32) | r1.x);
+          const float4* const frames = reinterpret_cast<const float4*>((static_cast<uint64_t>(r1.w) << 32) | r1.z);
+          L.enter(rec, p);
+          for (uint32_t r = 0; r < mesh->n_roots && !overflow; r++) {
+            if (lane == 0) lds_store(front, 0, make_uint2(mesh->roots4[r], 0u));
+            __syncthreads();
+            uint32_t fc = 1;
+            while (fc > 0 && !overflow) {
+              const uint32_t take = min(fc, 16u);
+              fc -= take;
+              uint2 e = make_uint2(kDone, 0u);
+              if (quad < take) e = lds_load(front, fc + quad);
+              __syncthreads();  // every quad has its entry before the pushes overwrite them
+              if (!(__uint_as_float(e.y) <= L.T)) e.x = kDone;
+              bool in = false;
+              uint2 child = make_uint2(kDone, 0u);
+              if (!(e.x & kRefLeaf) && e.x != kDone) {
+                const float4 c0 = nodes[8ull * e.x + 2 * q4], c1 = nodes[8ull * e.x + 2 * q4 + 1];
+                const float sc = box_score(L.q, c0.x, c0.y, c0.z, c0.w, c1.x, c1.y) * (1.0f - 4.0f * kU);
+                child = make_uint2(__float_as_uint(c1.z), __float_as_uint(sc));
+                in = (child.x != kDone) & (sc <= L.T);
+              }
+              const uint64_t need = __ballot(in);
+              const uint32_t more = static_cast<uint32_t>(__popcll(need));
+              if (fc + more > kPointFrontier) {
+                overflow = true;
+              } else if (in) {
+                lds_store(front, fc + static_cast<uint32_t>(__popcll(need & ((1ull << lane) - 1ull))), child);
+              }
+              fc += more;
+              if (e.x & kRefLeaf) {
+                uint32_t off, cnt;
+                leaf_range(e.x, mesh->bigleaf, off, cnt);
+                for (uint32_t s = off + q4; s < off + cnt; s += 4) L.test(frames, s, r0.x);
+              }
+              L.T = wave_min_f(L.T);
+              L.U = wave_min_f(L.U);
+              overflow = overflow || __ballot(L.full) != 0;
+              __syncthreads();
+            }
+          }
+        }
+      }
+      while (ref == kDone && st.sp > 0 && !overflow) {
+        const uint2 e = lds_load(top, --st.sp);
+        if (__uint_as_float(e.y) <= L.U) ref = e.x;
+      }
+    }
+    if (!overflow) {
+      const uint32_t c = L.left();
+      uint32_t total;
+      const uint32_t to_lane = wave_prefix(c, lane, &total);
+      uint2* to;
+      overflow = !scene_point_row(A, v, total, lane == 0, [](uint32_t at) { return __builtin_amdgcn_readfirstlane(at); }, to);
+      if (!overflow) L.write(to + to_lane);
+    }
+    if (overflow && lane == 0) A.rest[rest + atomicAdd(A.more_count, 1u)] = v;  // its row stays marked
+  }
+}
+
+// The candidates settled in FP64, one lane per point: the kernels' order of picks, so their results.
+__global__ __launch_bounds__(kBlock) void k_scene_point_resolve(SceneArgs A) {
+  const uint64_t v = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (v >= A.n) return;
+  const uint2* c = A.contenders + kSceneRow * v;
+  const uint2 c0 = c[0];
+  if (c0.x == kOverflow) return;  // left to the FP64 walk
+  uint32_t count = 0;
+  if (c0.x == kPooled) {
+    count = c[1].x;
+    c = A.contender_pool + c0.y;
+  } else {
+    while (count < kSceneRow && c[count].x != kNoHit) count++;
+  }
+  const uint64_t i = A.order ? A.order[v] : v;
+  const D3 p = d3(A.origins[3 * i], A.origins[3 * i + 1], A.origins[3 * i + 2]);
+  ScenePick b = {__builtin_huge_val(), kNoHit, kNoHit, kNoHit};
+  for (uint32_t k = 0; k < count; k++) {
+    const uint32_t slot = c[k].x, inst = c[k].y;
+    const float* W = A.world + 16ull * inst;
+    const Tri t = load_tri(A.meshes[A.instance_geometry[inst]].tris, slot);
+    const D3 q = closest_on_tri_d(p, world_vertex_f(W, t.p0), world_vertex_f(W, t.p1), world_vertex_f(W, t.p2));
+    const double d2 = ddist2(p, q);
+    const uint32_t face = t.face();
+    if (scene_pick_less(d2, inst, face, b)) b = {d2, inst, face, slot};
+  }
+  scene_point_out(A, i, false, b, p);
+}
+
+// ------------------------------------------------------------------------------------------
 // Scene closest point, one wave per point, for the points the four-lane kernel left (those whose
 // walks are long: a point near the centre of a closed mesh is close to every triangle). The wave
 // walks the top level together; in each instance it keeps an LDS frontier of 4-wide nodes: every
@@ -4060,29 +4517,14 @@ __device__ __forceinline__ void wave_min_pick(ScenePick& b) {
   }
 }
 
-__device__ __forceinline__ float wave_min_f(float v) {
-  for (int m = 1; m < 64; m <<= 1) v = fminf(v, __shfl_xor(v, m, 64));
-  return v;
-}
-
-// Exclusive prefix sum of c over the wave; *total receives the sum.
-__device__ __forceinline__ uint32_t wave_prefix(uint32_t c, uint32_t lane, uint32_t* total) {
-  uint32_t x = c;
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t y = __shfl_up(x, d, 64);
-    if (lane >= static_cast<uint32_t>(d)) x += y;
-  }
-  *total = __shfl(x, 63, 64);
-  return x - c;
-}
-
 __global__ __launch_bounds__(64) void k_scene_closest_point_wide(SceneArgs A) {
   __shared__ uint2 front[kWideFrontier];
   __shared__ uint2 top[kTlasStack];
   const uint32_t lane = threadIdx.x;
-  const uint32_t nh = *A.heavy_count;
+  const uint32_t nh = A.rest ? *A.more_count : *A.heavy_count;
+  const uint32_t* const list = A.rest ? A.rest + *A.rest_count : A.heavy;
   for (uint32_t h = blockIdx.x; h < nh; h += gridDim.x) {
-    const uint64_t i = A.heavy[h];
+    const uint64_t i = A.rest && A.order ? A.order[list[h]] : list[h];
     const float px = A.origins[3 * i], py = A.origins[3 * i + 1], pz = A.origins[3 * i + 2];
     const D3 p = d3(px, py, pz);
     ScenePick b = {__builtin_huge_val(), kNoHit, kNoHit, kNoHit};
@@ -4334,14 +4776,14 @@ hipError_t launch_batch_raycast_first(const BatchArgs& a, uint32_t stack_lds, ui
   return hipGetLastError();
 }
 
-__global__ void k_scene_ray_reset(uint32_t* queue, uint32_t* count, uint32_t* pool_count) {
+__global__ void k_scene_reset(uint32_t* queue, uint32_t* count, uint32_t* pool_count) {
   if (threadIdx.x < kWalkQueues) queue[32 * threadIdx.x] = 0u;
   if (threadIdx.x == 0) *count = *pool_count = 0u;
 }
 
 hipError_t launch_scene_raycast_first4(const SceneArgs& a, uint64_t quads, hipStream_t s) {
   if (a.n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scene_ray_reset, dim3(1), dim3(64), 0, s, a.queue, a.heavy_count,
+  hipLaunchKernelGGL(k_scene_reset, dim3(1), dim3(64), 0, s, a.queue, a.heavy_count,
                      a.contender_pool_count);
   hipLaunchKernelGGL(k_scene_raycast_first4, dim3(static_cast<uint32_t>(quads / (kBlock / 4))), dim3(kBlock), 0, s, a);
   hipLaunchKernelGGL(k_scene_ray_resolve, dim3(static_cast<uint32_t>((a.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a);
@@ -4368,14 +4810,35 @@ hipError_t launch_scene_closest_point(const SceneArgs& a, uint64_t threads, hipS
 
 hipError_t launch_scene_closest_point4(const SceneArgs& a, uint64_t threads, hipStream_t s) {
   if (a.n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, a.queue);
-  if (a.heavy) hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, a.heavy_count);
-  hipLaunchKernelGGL(k_scene_closest_point4, dim3(static_cast<uint32_t>(threads / kBlock)), dim3(kBlock), 0, s, a);
+  if (!a.rest) {  // otherwise the FP32 walk's launch cleared them
+    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, a.queue);
+    if (a.heavy) hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, a.heavy_count);
+  }
+  const dim3 grid(static_cast<uint32_t>(threads / kBlock));
+  if (a.rest)
+    hipLaunchKernelGGL(k_scene_closest_point4<true>, grid, dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_scene_closest_point4<false>, grid, dim3(kBlock), 0, s, a);
+  return hipGetLastError();
+}
+
+__global__ void k_scene_point_reset(SceneArgs A) {
+  if (threadIdx.x < kWalkQueues) A.queue[32 * threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *A.heavy_count = *A.rest_count = *A.more_count = *A.contender_pool_count = *A.rest_queue = 0u;
+}
+
+hipError_t launch_scene_point_walk4(const SceneArgs& a, uint64_t quads, hipStream_t s) {
+  if (a.n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_scene_point_reset, dim3(1), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(k_scene_point_walk4, dim3(static_cast<uint32_t>(quads / (kBlock / 4))), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(k_scene_point_wide, dim3(static_cast<uint32_t>(a.n < kScenePointWaves ? a.n : kScenePointWaves)), dim3(64), 0,
+                     s, a);
+  hipLaunchKernelGGL(k_scene_point_resolve, dim3(static_cast<uint32_t>((a.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_scene_closest_point_wide(const SceneArgs& a, uint32_t waves, hipStream_t s) {
-  if (a.n == 0 || !a.heavy) return hipSuccess;
+  if (a.n == 0 || !(a.heavy || a.rest)) return hipSuccess;
   hipLaunchKernelGGL(k_scene_closest_point_wide, dim3(waves), dim3(64), 0, s, a);
   return hipGetLastError();
 }
