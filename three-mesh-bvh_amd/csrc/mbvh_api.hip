@@ -113,7 +113,8 @@ struct mbvh_batch {
   uint32_t* d_counter = nullptr;  // work-queue counter
   uint32_t max_stack = 0;
   uint32_t max_stack4 = 0;
-  mbvh_batch_tuning tuning{4, 16, 256, 4, 0.0f};
+  bool tuned = false;  // `tuning` was measured by mbvh_batch_autotune
+  mbvh_batch_tuning tuning{4, 16, 64, 4, 0.0f};
 };
 
 struct mbvh_batch_graph {
@@ -2199,6 +2200,16 @@ int check_batch_call(const char* fn, const mbvh_ctx* ctx, const mbvh_batch* b, c
   return MBVH_OK;
 }
 
+// The shape of a launch whose caller names none: the autotuned one, else by the number of rays. One lane
+// per ray and work items of one wave are the fastest from a wave's worth of rays on, four lanes below
+// (microseconds for 16 / 64 / 1,000 / 65,536 / 1,048,576 / 4,194,304 rays on 64 meshes of up to 50,000 triangles:
+// one lane 68 / 84 / 126 / 221 / 499 / 1,499; four lanes 54 / 114 / 141 / 253 / 709 / 2,577, and with
+// items of 256 rays 54 / 114 / 410 / 682 / 938 / 2,743), where the trees fit its stack.
+mbvh_batch_tuning tuning_for(const mbvh_ctx* ctx, const mbvh_batch* b, uint64_t n) {
+  if (b->tuned || n < 64 || b->max_stack > 8 + ctx->stack_ovf_entries) return b->tuning;
+  return {1, 8, 64, 4, 0.0f};
+}
+
 int enqueue_batch(mbvh_ctx* ctx, mbvh_batch* b, const BatchCall& c, const mbvh_batch_tuning& t, hipStream_t s) {
   const bool local = c.windows != nullptr;
   const uint32_t* order = nullptr;
@@ -2317,7 +2328,7 @@ extern "C" int mbvh_batch_raycast_first_d(mbvh_ctx* ctx, mbvh_batch* batch, cons
   MBVH_BATCH_CALL;
   int rc = check_batch_call(fn, ctx, batch, c);
   if (rc) return rc;
-  const mbvh_batch_tuning t = tuning ? *tuning : batch->tuning;
+  const mbvh_batch_tuning t = tuning ? *tuning : tuning_for(ctx, batch, c.n);
   if ((rc = check_tuning(fn, t))) return rc;
   if ((rc = set_device(ctx))) return rc;
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
@@ -2359,7 +2370,7 @@ extern "C" int mbvh_batch_raycast_first(mbvh_ctx* ctx, mbvh_batch* batch, const 
                     far_dist, static_cast<uint32_t*>(oF), static_cast<float*>(oT), static_cast<float*>(oP),
                     static_cast<float*>(oB), ctx->grad_ws.ptr, ctx->grad_ws.bytes};
   if ((rc = check_batch_call(fn, ctx, batch, c))) return rc;
-  if ((rc = enqueue_batch(ctx, batch, c, batch->tuning, s))) return rc;
+  if ((rc = enqueue_batch(ctx, batch, c, tuning_for(ctx, batch, c.n), s))) return rc;
   MBVH_HIP(hipMemcpyAsync(face_index, oF, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   if (distance) MBVH_HIP(hipMemcpyAsync(distance, oT, n * sizeof(float), hipMemcpyDeviceToHost, s));
   if (point) MBVH_HIP(hipMemcpyAsync(point, oP, v3, hipMemcpyDeviceToHost, s));
@@ -2413,7 +2424,7 @@ extern "C" int mbvh_batch_raycast_first_local_f64(mbvh_ctx* ctx, mbvh_batch* bat
               static_cast<float*>(oP), static_cast<float*>(oB), ctx->grad_ws.ptr, ctx->grad_ws.bytes,
               static_cast<float*>(dOl), static_cast<float*>(dDl), static_cast<float*>(dWn)};
   if ((rc = check_batch_call(fn, ctx, batch, c))) return rc;
-  if ((rc = enqueue_batch(ctx, batch, c, batch->tuning, s))) return rc;
+  if ((rc = enqueue_batch(ctx, batch, c, tuning_for(ctx, batch, c.n), s))) return rc;
   MBVH_HIP(hipMemcpyAsync(face_index, oF, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   if (distance) MBVH_HIP(hipMemcpyAsync(distance, oT, n * sizeof(float), hipMemcpyDeviceToHost, s));
   if (point) MBVH_HIP(hipMemcpyAsync(point, oP, v3, hipMemcpyDeviceToHost, s));
@@ -2471,6 +2482,7 @@ extern "C" int mbvh_batch_autotune(mbvh_ctx* ctx, mbvh_batch* batch, const float
   (void)hipEventDestroy(e1);
   if (rc) return rc;
   batch->tuning = best;
+  batch->tuned = true;
   *out_tuning = best;
   return MBVH_OK;
 }
@@ -2489,7 +2501,7 @@ extern "C" int mbvh_batch_graph_create(mbvh_ctx* ctx, mbvh_batch* batch, const f
   MBVH_BATCH_CALL;
   int rc = check_batch_call(fn, ctx, batch, c);
   if (rc) return rc;
-  const mbvh_batch_tuning t = tuning ? *tuning : batch->tuning;
+  const mbvh_batch_tuning t = tuning ? *tuning : tuning_for(ctx, batch, c.n);
   if ((rc = check_tuning(fn, t))) return rc;
   std::lock_guard<std::mutex> guard(ctx->lock);
   if ((rc = set_device(ctx))) return rc;
