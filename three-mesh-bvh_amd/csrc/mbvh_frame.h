@@ -54,6 +54,13 @@ __device__ __forceinline__ D3f f_cross(D3f a, D3f b) {
 }
 __device__ __forceinline__ D3f f_scale(D3f a, double s) { return {a.x * s, a.y * s, a.z * s}; }
 
+// 1 / sqrt(x) to 2^-44 of its value, far below the float rounding of what it scales: the hardware's
+// estimate (2^-23) and one Newton step.
+__device__ __forceinline__ double f_rsqrt(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  return r * (1.5 - 0.5 * x * r * r);
+}
+
 __device__ __forceinline__ void tri_frame(f3 fa, f3 fb, f3 fc, float4* out) {
   const D3f a = {fa.x, fa.y, fa.z}, b = {fb.x, fb.y, fb.z}, c = {fc.x, fc.y, fc.z};
   const D3f ab = f_sub(b, a), bc = f_sub(c, b), ca = f_sub(a, c);
@@ -72,32 +79,36 @@ __device__ __forceinline__ void tri_frame(f3 fa, f3 fb, f3 fc, float4* out) {
     w = f_sub(b, c);
     ll = l2;
   }
-  const double L = sqrt(ll);
   D3f u = {1, 0, 0}, v = {0, 1, 0}, n = {0, 0, 1};
-  double cx = 0, cy = 0;
-  if (L > 0) {
-    u = f_scale(base, 1 / L);
+  double L = 0, cx = 0, cy = 0;
+  if (!(ll == 0)) {
+    const double r = f_rsqrt(ll);
+    L = ll * r;
+    u = f_scale(base, r);
     n = f_cross(u, w);
-    const double h = sqrt(f_dot(n, n));
-    if (h > 0) {
-      n = f_scale(n, 1 / h);
-    } else {  // collinear: any normal
+    double hh = f_dot(n, n);
+    if (hh == 0) {  // collinear: any normal
       n = f_cross(u, fabs(u.x) < 0.6 ? D3f{1, 0, 0} : D3f{0, 1, 0});
-      n = f_scale(n, 1 / sqrt(f_dot(n, n)));
+      hh = f_dot(n, n);
     }
+    n = f_scale(n, f_rsqrt(hh));
     v = f_cross(n, u);
     cx = f_dot(u, w);
     cy = f_dot(v, w);
   }
-  const double m1 = sqrt((cx - L) * (cx - L) + cy * cy), m2 = sqrt(cx * cx + cy * cy);
-  double e1x = 0, e1y = 1, e2x = 1, e2y = 0;
-  if (m1 > 0) {
-    e1x = (cx - L) / m1;
-    e1y = cy / m1;
+  const double x1 = cx - L, mm1 = x1 * x1 + cy * cy, mm2 = cx * cx + cy * cy;
+  double m1 = 0, m2 = 0, e1x = 0, e1y = 1, e2x = 1, e2y = 0;
+  if (!(mm1 == 0)) {
+    const double r = f_rsqrt(mm1);
+    m1 = mm1 * r;
+    e1x = x1 * r;
+    e1y = cy * r;
   }
-  if (m2 > 0) {
-    e2x = cx / m2;
-    e2y = cy / m2;
+  if (!(mm2 == 0)) {
+    const double r = f_rsqrt(mm2);
+    m2 = mm2 * r;
+    e2x = cx * r;
+    e2y = cy * r;
   }
   const float wide = static_cast<float>(256.0 * 5.9604644775390625e-08 * 1.0001 * ll);
   const bool flat = cy <= L * 9.5367431640625e-07;  // 2^-20; false for NaN, whose w is NaN already

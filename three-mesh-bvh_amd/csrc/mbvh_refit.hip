@@ -68,19 +68,43 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_bound(RefitArgs a) {
   }
 }
 
-// One lane per slot: its three corners gathered, and its frame from them.
+// A block's slots: one lane per corner gathers it, then one lane per slot makes its frame. Corners and
+// frames go through LDS, so that every wave reads and writes whole lines (800,000 slots: 32 us, as
+// long as a copy of as many bytes; 41 with each lane gathering its corners and writing its frame in place;
+// 18 without frames).
 __global__ __launch_bounds__(kRefitBlock) void k_refit_tris(RefitArgs a) {
+  __shared__ float4 rows[kFrameRows * kRefitBlock];
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kRefitBlock;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x; i < a.n_slots; i += stride) {
-    float4 r[3];
-    for (int k = 0; k < 3; k++) {
-      const float* p = a.positions + static_cast<uint64_t>(a.vidx[3 * i + k]) * a.stride + a.offset;
-      r[k] = make_float4(p[0], p[1], p[2], a.tris[3 * i + k].w);
+  for (uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * kRefitBlock; i0 < a.n_slots; i0 += stride) {
+    const uint64_t left = a.n_slots - i0;
+    const uint32_t n = static_cast<uint32_t>(left < kRefitBlock ? left : kRefitBlock);
+    float4 c[3];
+#pragma unroll
+    for (uint32_t j = 0; j < 3; j++) {
+      const uint32_t k = threadIdx.x + j * kRefitBlock;
+      if (k >= 3 * n) continue;
+      const float* p = a.positions + static_cast<uint64_t>(a.vidx[3 * i0 + k]) * a.stride + a.offset;
+      c[j] = make_float4(p[0], p[1], p[2], a.tris[3 * i0 + k].w);
     }
-    for (int k = 0; k < 3; k++) a.tris[3 * i + k] = r[k];
+#pragma unroll
+    for (uint32_t j = 0; j < 3; j++) {
+      const uint32_t k = threadIdx.x + j * kRefitBlock;
+      if (k >= 3 * n) continue;
+      a.tris[3 * i0 + k] = c[j];
+      rows[k] = c[j];
+    }
+    __syncthreads();
     float4 f[kFrameRows];
-    tri_frame(mk(r[0].x, r[0].y, r[0].z), mk(r[1].x, r[1].y, r[1].z), mk(r[2].x, r[2].y, r[2].z), f);
-    for (int k = 0; k < kFrameRows; k++) a.frames[kFrameRows * i + k] = f[k];
+    if (threadIdx.x < n) {
+      const float4 p = rows[3 * threadIdx.x], q = rows[3 * threadIdx.x + 1], r = rows[3 * threadIdx.x + 2];
+      tri_frame(mk(p.x, p.y, p.z), mk(q.x, q.y, q.z), mk(r.x, r.y, r.z), f);
+    }
+    __syncthreads();
+    if (threadIdx.x < n)
+      for (int k = 0; k < kFrameRows; k++) rows[kFrameRows * threadIdx.x + k] = f[k];
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < kFrameRows * n; k += kRefitBlock) a.frames[kFrameRows * i0 + k] = rows[k];
+    __syncthreads();
   }
 }
 
@@ -118,7 +142,8 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_leaves(RefitArgs a) {
     const uint32_t cnt = w[7] & 0xFFFFu;  // u16[14]: count (u16[15] is the leaf flag)
     float b[6] = {inf, inf, inf, -inf, -inf, -inf};
     for (uint64_t c = 3ull * off; c < 3ull * (static_cast<uint64_t>(off) + cnt); c++) {
-      const float* p = a.positions + static_cast<uint64_t>(a.vidx[c]) * a.stride + a.offset;
+      const float4 t = a.tris[c];  // k_refit_tris gathered it: one load instead of four
+      const float p[3] = {t.x, t.y, t.z};
       for (int k = 0; k < 3; k++) {
         if (p[k] < b[k]) b[k] = p[k];
         if (p[k] > b[3 + k]) b[3 + k] = p[k];
@@ -133,28 +158,47 @@ __global__ __launch_bounds__(kRefitBlock) void k_refit_leaves(RefitArgs a) {
 }
 
 // The internal nodes of one depth, whose children were decided by earlier launches.
+__device__ __forceinline__ void refit_node(const RefitArgs& a, uint64_t node) {
+  if (a.node_ids && !(a.changed[node] & kRefitVisit)) {
+    a.changed[node] = 0u;
+    return;
+  }
+  const uint64_t left = node + 1;
+  const uint64_t right = node + a.ref_nodes[8 * node + 6];
+  const bool any = ((a.changed[left] | a.changed[right]) & kRefitChanged) != 0u;
+  if (any) {
+    const float* lb = reinterpret_cast<const float*>(a.ref_nodes + 8 * left);
+    const float* rb = reinterpret_cast<const float*>(a.ref_nodes + 8 * right);
+    float u[6];
+    for (int k = 0; k < 3; k++) {
+      u[k] = lb[k] < rb[k] ? lb[k] : rb[k];
+      u[3 + k] = lb[3 + k] > rb[3 + k] ? lb[3 + k] : rb[3 + k];
+    }
+    put_box(a, node, u);
+  }
+  a.changed[node] = any ? kRefitChanged : 0u;
+}
+
 __global__ __launch_bounds__(kRefitBlock) void k_refit_level(RefitArgs a, const uint32_t* nodes, uint64_t count) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kRefitBlock;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x; i < count; i += stride) {
-    const uint64_t node = nodes[i];
-    if (a.node_ids && !(a.changed[node] & kRefitVisit)) {
-      a.changed[node] = 0u;
-      continue;
-    }
-    const uint64_t left = node + 1;
-    const uint64_t right = node + a.ref_nodes[8 * node + 6];
-    const bool any = ((a.changed[left] | a.changed[right]) & kRefitChanged) != 0u;
-    if (any) {
-      const float* lb = reinterpret_cast<const float*>(a.ref_nodes + 8 * left);
-      const float* rb = reinterpret_cast<const float*>(a.ref_nodes + 8 * right);
-      float u[6];
-      for (int k = 0; k < 3; k++) {
-        u[k] = lb[k] < rb[k] ? lb[k] : rb[k];
-        u[3 + k] = lb[3 + k] > rb[3 + k] ? lb[3 + k] : rb[3 + k];
-      }
-      put_box(a, node, u);
-    }
-    a.changed[node] = any ? kRefitChanged : 0u;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRefitBlock + threadIdx.x; i < count; i += stride)
+    refit_node(a, nodes[i]);
+}
+
+// A run of depths of at most kSmallLevel nodes each, deepest first, in one workgroup with a barrier between
+// depths: a launch each (4.5 us) is longer than their work. 800,000 triangles, 19 depths: 58 us against 86.
+constexpr uint32_t kSmallLevel = 1024;
+constexpr uint32_t kSmallRun = 48;
+struct RefitRun {
+  uint32_t n;
+  uint32_t off[kSmallRun + 1];  // from a.levels + base: depth j of the run is off[j] .. off[j + 1]
+};
+__global__ __launch_bounds__(kSmallLevel) void k_refit_small(RefitArgs a, const uint32_t* nodes, RefitRun run) {
+  for (uint32_t j = run.n; j-- > 0;) {
+    const uint32_t i = run.off[j] + threadIdx.x;
+    if (i < run.off[j + 1]) refit_node(a, nodes[i]);
+    __threadfence_block();
+    __syncthreads();
   }
 }
 
@@ -320,6 +364,16 @@ hipError_t launch_refit(const RefitArgs& a, hipStream_t s) {
   if (a.n_leaves) hipLaunchKernelGGL(k_refit_leaves, dim3(blocks_for(a.n_leaves)), dim3(kRefitBlock), 0, s, a);
   for (uint32_t d = a.n_levels; d-- > 0;) {
     const uint64_t count = a.level_off[d + 1] - a.level_off[d];
+    // the depths from d up that are small as well
+    uint32_t first = d + 1;
+    while (first > 0 && d + 1 - first < kSmallRun && a.level_off[first] - a.level_off[first - 1] <= kSmallLevel) first--;
+    if (d + 1 - first > 1) {
+      RefitRun run{d + 1 - first, {}};
+      for (uint32_t j = 0; j <= run.n; j++) run.off[j] = static_cast<uint32_t>(a.level_off[first + j] - a.level_off[first]);
+      hipLaunchKernelGGL(k_refit_small, dim3(1), dim3(kSmallLevel), 0, s, a, a.levels + a.level_off[first], run);
+      d = first;
+      continue;
+    }
     if (count)
       hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(count)), dim3(kRefitBlock), 0, s, a, a.levels + a.level_off[d],
                          count);
