@@ -29,7 +29,30 @@ def _soup(rng, n, size, spread, thin):
     return np.stack([a, a + e, a + e * rng.uniform(-0.5, 1.5, (n, 1)) + rng.standard_normal((n, 3)) * size * thin], 1)
 
 
+def collinear(n):
+    """n exactly collinear triangles (corners a, a + e, a + 2 e in any order, whole numbers) 16 apart, a
+    triangle at least 1.25 from each one's middle, and queries within 0.5 of the middles: (triangles, queries,
+    distances). All products are exact in FP32, so the exact step has no noise either."""
+    rng = np.random.default_rng(32)
+    side = int(np.ceil(n ** (1 / 3)))
+    mid = 16.0 * np.stack(np.unravel_index(np.arange(n), (side,) * 3), 1)
+    e = rng.integers(-3, 4, (n, 3)).astype(float)
+    e[:, 0] = 1 + rng.integers(0, 3, n)
+    line = np.stack([mid - e, mid, mid + e], 1)
+    line = np.stack([x[rng.permutation(3)] for x in line])
+    axis = rng.integers(0, 3, n)
+    other = mid[:, None, :] + rng.integers(-2, 3, (n, 3, 3))
+    other[np.arange(n), 0, (axis + 1) % 3] += 4
+    other[np.arange(n), 1, (axis + 2) % 3] += 4
+    other[np.arange(n), :, axis] = mid[np.arange(n), axis][:, None] + 1.5
+    off = 0.25 * rng.integers(-1, 2, (n, 3))
+    t = np.clip((off * e).sum(1) / (e * e).sum(1), -1, 1)
+    return np.concatenate([line, other]), mid + off, np.linalg.norm(off - t[:, None] * e, axis=1)
+
+
 def _cases(name):
+    if name == "line":
+        return collinear(1000)[:2]
     rng = np.random.default_rng(31)
     if name.startswith("few"):  # a leaf alone: odd and even counts of the two-triangle step
         t = _soup(rng, int(name[3:]), 1.0, 2.0, 1.0)
@@ -38,7 +61,7 @@ def _cases(name):
         t = np.concatenate([_soup(rng, 400, 0.5, 2.0, 10.0 ** -k) for k in range(0, 8)])
         flat = _soup(rng, 90, 0.5, 2.0, 1.0)
         flat[:30, 1] = flat[:30, 0]                       # two equal corners
-        flat[30:60, 2] = 0.5 * (flat[30:60, 0] + flat[30:60, 1])  # collinear
+        flat[30:60, 2] = 0.5 * (flat[30:60, 0] + flat[30:60, 1])  # collinear up to the corners' rounding
         flat[60:, 1:] = flat[60:, :1]                     # a point
         return np.concatenate([t, flat]), rng.uniform(-3, 3, (4099, 3))
     if name == "fan":  # the closest feature of every query above the tip is the vertex all 96 share
@@ -64,7 +87,7 @@ def _cases(name):
     raise KeyError(name)
 
 
-@pytest.mark.parametrize("name", ["few1", "few2", "few3", "few9", "few11", "thin", "fan", "twice", "far", "on"])
+@pytest.mark.parametrize("name", ["few1", "few2", "few3", "few9", "few11", "thin", "fan", "twice", "far", "on", "line"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("max_t", [float("inf"), 0.7])
 def test_frames(ctx, name, dtype, max_t):

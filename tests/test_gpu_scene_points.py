@@ -8,6 +8,7 @@ import pytest
 import mbvh_amd as M
 from mbvh_amd import geometry as G
 from helpers import build_mesh
+from test_gpu_closest_frames import collinear
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +113,24 @@ def test_not_finite(setup):
     p[0::8, 0], p[1::8, 1], p[2::8] = np.nan, np.inf, -np.inf
     ref = check(setup, matrices(3, rng), [0, 1, 2], p)
     assert np.all(ref["face"][0::8] == M.NO_HIT) and np.all(ref["face"][3::8] != M.NO_HIT)
+
+
+def test_collinear(setup):
+    """Exactly collinear triangles are the nearest (moved by whole numbers and doubled, so still exactly so)."""
+    ctx, _ = setup
+    tris, local, dist = collinear(1000)
+    pos = tris.astype(np.float32).reshape(-1, 3)
+    g, idx, tree = build_mesh(G.Geometry(pos, np.arange(len(pos), dtype=np.uint32)))
+    mesh = ctx.upload(tree, g.positions, idx)
+    m = np.stack([np.eye(4), np.diag([2.0, 2.0, 2.0, 1.0])])
+    m[1, :3, 3] = 512
+    world = np.ascontiguousarray(m.transpose(0, 2, 1).reshape(-1, 16), dtype=np.float32)
+    inverse = np.linalg.inv(world.reshape(-1, 4, 4).astype(np.float64)).reshape(-1, 16).astype(np.float32)
+    sc = ctx.scene([mesh], world, inverse, np.zeros(2, np.uint32))
+    points = np.concatenate([local, 2 * local + 512]).astype(np.float32)
+    got = sc.closest_point(np.tile(points, (LEAST // len(points), 1)))
+    want = np.tile(np.concatenate([dist, 2 * dist]), LEAST // len(points))
+    np.testing.assert_allclose(got["distance"], want, rtol=1e-6)
+    assert np.array_equal(got["instance"], np.tile(np.repeat([0, 1], 1000), LEAST // len(points)))
+    sc.free()
+    mesh.free()

@@ -29,10 +29,14 @@
 // of 128 k, from 2 d L <= d^2 + L^2 and coarser steps, lists six candidates per query instead of two on
 // a 256^3 grid over a million-triangle sphere: 317 ms instead of the figures at the kernels.)
 //
-// w is negative when the triangle is degenerate to within 2^-20 (apex height under 2^-20 L, or L = 0):
-// the exact closest point can then be NaN (0 / 0 weights) and the triangle never win, so its distance
-// may be listed but must not bound the search. w is NaN when a vertex is: every comparison with its
-// bounds fails, and the triangle is left to the exact step.
+// A triangle whose apex height is at most 2^-20 L has the frame of its base alone, with any normal: the
+// cross product that would give the normal is rounding noise there (for collinear corners u x w has its
+// whole value from u's rounding), and a frame from it is not orthogonal. The triangle holds its base and
+// lies within that height of it, so its distance is at most that of the base and at least that less the
+// height: 2 d h <= 32 k d L more on one side, in all 33.5 k d^2 + 508 k L^2, w = 512 k L^2. Its w is negative:
+// the exact closest point can be NaN (0 / 0 weights) or, the signs that choose its region being rounding noise,
+// not the closest, so the triangle is listed but must not bound the search. w is NaN where a corner is not
+// finite, and d2 too: every comparison with its bounds fails, and the triangle is left to the exact step.
 #pragma once
 
 #include "mbvh_device.h"
@@ -81,20 +85,24 @@ __device__ __forceinline__ void tri_frame(f3 fa, f3 fb, f3 fc, float4* out) {
   }
   D3f u = {1, 0, 0}, v = {0, 1, 0}, n = {0, 0, 1};
   double L = 0, cx = 0, cy = 0;
+  bool flat = true;
   if (!(ll == 0)) {
     const double r = f_rsqrt(ll);
     L = ll * r;
     u = f_scale(base, r);
     n = f_cross(u, w);
     double hh = f_dot(n, n);
-    if (hh == 0) {  // collinear: any normal
+    flat = hh <= 9.094947017729282e-13 * ll;  // 2^-40
+    if (flat) {
       n = f_cross(u, fabs(u.x) < 0.6 ? D3f{1, 0, 0} : D3f{0, 1, 0});
       hh = f_dot(n, n);
     }
     n = f_scale(n, f_rsqrt(hh));
     v = f_cross(n, u);
-    cx = f_dot(u, w);
-    cy = f_dot(v, w);
+    if (!flat) {
+      cx = f_dot(u, w);
+      cy = f_dot(v, w);
+    }
   }
   const double x1 = cx - L, mm1 = x1 * x1 + cy * cy, mm2 = cx * cx + cy * cy;
   double m1 = 0, m2 = 0, e1x = 0, e1y = 1, e2x = 1, e2y = 0;
@@ -110,10 +118,10 @@ __device__ __forceinline__ void tri_frame(f3 fa, f3 fb, f3 fc, float4* out) {
     e2x = cx * r;
     e2y = cy * r;
   }
-  const float wide = static_cast<float>(256.0 * 5.9604644775390625e-08 * 1.0001 * ll);
-  const bool flat = cy <= L * 9.5367431640625e-07;  // 2^-20; false for NaN, whose w is NaN already
+  const float wide = static_cast<float>((flat ? 512.0 : 256.0) * 5.9604644775390625e-08 * 1.0001 * ll);
+  const float f0w = l0 + l1 + l2 < 1e300 ? (flat ? -wide : wide) : __builtin_nanf("");
   // p0 is one of the float vertices: the conversion is exact
-  out[0] = make_float4(static_cast<float>(p0.x), static_cast<float>(p0.y), static_cast<float>(p0.z), flat ? -wide : wide);
+  out[0] = make_float4(static_cast<float>(p0.x), static_cast<float>(p0.y), static_cast<float>(p0.z), f0w);
   out[1] = make_float4(static_cast<float>(u.x), static_cast<float>(u.y), static_cast<float>(u.z), static_cast<float>(L));
   out[2] = make_float4(static_cast<float>(v.x), static_cast<float>(v.y), static_cast<float>(v.z), static_cast<float>(e1x));
   out[3] = make_float4(static_cast<float>(n.x), static_cast<float>(n.y), static_cast<float>(n.z), static_cast<float>(e1y));
