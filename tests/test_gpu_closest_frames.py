@@ -50,9 +50,22 @@ def collinear(n):
     return np.concatenate([line, other]), mid + off, np.linalg.norm(off - t[:, None] * e, axis=1)
 
 
+def segments(order, n=3000):
+    """Strands of n segments stored as triangles with two equal corners ("abb", "aba" or "aab")."""
+    rng = np.random.default_rng(33)
+    p = np.cumsum(np.concatenate([rng.uniform(-2, 2, (n // 100, 1, 3)), 0.1 * rng.standard_normal((n // 100, 100, 3))], 1), 1)
+    ends = dict(a=p[:, :-1].reshape(-1, 3), b=p[:, 1:].reshape(-1, 3))
+    return np.stack([ends[c] for c in order], 1).astype(np.float32)
+
+
 def _cases(name):
     if name == "line":
         return collinear(1000)[:2]
+    if name == "lines":  # none of the triangles bounds the search
+        tris, q, _ = collinear(1000)
+        return tris[:1000], q
+    if name in ("abb", "aba", "aab"):
+        return segments(name), np.random.default_rng(34).uniform(-3, 3, (4099, 3))
     rng = np.random.default_rng(31)
     if name.startswith("few"):  # a leaf alone: odd and even counts of the two-triangle step
         t = _soup(rng, int(name[3:]), 1.0, 2.0, 1.0)
@@ -87,7 +100,7 @@ def _cases(name):
     raise KeyError(name)
 
 
-@pytest.mark.parametrize("name", ["few1", "few2", "few3", "few9", "few11", "thin", "fan", "twice", "far", "on", "line"])
+@pytest.mark.parametrize("name", ["few1", "few2", "few3", "few9", "few11", "thin", "fan", "twice", "far", "on", "line", "lines", "abb", "aba", "aab"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("max_t", [float("inf"), 0.7])
 def test_frames(ctx, name, dtype, max_t):

@@ -8,7 +8,7 @@ import pytest
 import mbvh_amd as M
 from mbvh_amd import geometry as G
 from helpers import build_mesh
-from test_gpu_closest_frames import collinear
+from test_gpu_closest_frames import collinear, segments
 
 pytestmark = pytest.mark.gpu
 
@@ -132,5 +132,33 @@ def test_collinear(setup):
     want = np.tile(np.concatenate([dist, 2 * dist]), LEAST // len(points))
     np.testing.assert_allclose(got["distance"], want, rtol=1e-6)
     assert np.array_equal(got["instance"], np.tile(np.repeat([0, 1], 1000), LEAST // len(points)))
+    sc.free()
+    mesh.free()
+
+
+@pytest.mark.parametrize("corners", ["abb", "aba", "aab"])
+def test_segments(setup, corners):
+    """Instances whose triangles all have two equal corners. Where those are a, a, b the closest point only
+    exists for points that a is nearest to (elsewhere it is 0 / 0), and no triangle bounds the walk."""
+    ctx, _ = setup
+    tris = segments(corners, 300)
+    pos = tris.reshape(-1, 3)
+    g, idx, tree = build_mesh(G.Geometry(pos, np.arange(len(pos), dtype=np.uint32)))
+    mesh = ctx.upload(tree, g.positions, idx)
+    rng = np.random.default_rng(9)
+    m = matrices(3, rng, span=3.0)
+    world = np.ascontiguousarray(m.transpose(0, 2, 1).reshape(-1, 16), dtype=np.float32)
+    inverse = np.linalg.inv(world.reshape(-1, 4, 4).astype(np.float64)).reshape(-1, 16).astype(np.float32)
+    sc = ctx.scene([mesh], world, inverse, np.zeros(3, np.uint32))
+    q = rng.uniform(-6, 6, (2000, 3)).astype(np.float32)
+    got = sc.closest_point(np.tile(q, (LEAST // 2000, 1)))
+    w = world.reshape(3, 4, 4).astype(np.float64)
+    a, b = (np.concatenate([tris[:, corners.index(c)].astype(np.float64) @ x[:3, :3] + x[3, :3] for x in w]) for c in "ab")
+    e = b - a
+    t = ((q.astype(np.float64) @ e.T) - (a * e).sum(1)) / (e * e).sum(1)
+    d = np.linalg.norm(q[:, None] - a - np.clip(t, 0, 1)[:, :, None] * e, axis=2)
+    if corners == "aab":
+        d[t > 0] = np.inf
+    np.testing.assert_allclose(got["distance"], np.tile(d.min(1), LEAST // 2000), rtol=1e-6)
     sc.free()
     mesh.free()

@@ -1272,9 +1272,9 @@ int closest_point_impl(mbvh_ctx* ctx, const mbvh_mesh* mesh, const float* q, uin
       a.tiles = std::min(chunk_tiles, tiles_total - t0);
       MBVH_HIP(launch_closest_point_packet(a, launch_threads(a.tiles * 64, ctx->max_threads), s));
       ClosestPointArgs r = a;
-      // rare (only when the candidate pool runs out): a small grid, whose waves leave at once when
-      // the redo count is 0
-      const uint64_t rt = launch_threads(4 * std::min<uint64_t>(a.tiles * 64, 4096), ctx->max_threads);
+      // rare (the candidate pool ran out, or a mesh of flat triangles that bound no search): its waves
+      // leave at once when the redo count is 0
+      const uint64_t rt = launch_threads(4 * std::min<uint64_t>(a.tiles * 64, 65536), ctx->max_threads);
       r.stack = stack_of(ctx, rt / 4);
       r.order = a.redo;
       r.n_dev = a.redo_count;

@@ -33,9 +33,14 @@
 // cross product that would give the normal is rounding noise there (for collinear corners u x w has its
 // whole value from u's rounding), and a frame from it is not orthogonal. The triangle holds its base and
 // lies within that height of it, so its distance is at most that of the base and at least that less the
-// height: 2 d h <= 32 k d L more on one side, in all 33.5 k d^2 + 508 k L^2, w = 512 k L^2. Its w is negative:
-// the exact closest point can be NaN (0 / 0 weights) or, the signs that choose its region being rounding noise,
-// not the closest, so the triangle is listed but must not bound the search. w is NaN where a corner is not
+// height: 2 d h <= 32 k d L more on one side, in all 33.5 k d^2 + 508 k L^2, w = 512 k L^2. With two equal
+// corners the triangle is the base and w stays 256 k L^2.
+//
+// The sign bit of w: the exact step may not reach the triangle's distance, so it may be listed but must not
+// bound the search. So where the corners are a, a, c, whose weights on the edge a a are 0 / 0, and where
+// three distinct corners are flat: the signs that choose the region are rounding noise then, and the face
+// region can divide one noise by another. a, b, b and a, b, a are sure: with d3 = d5 and d4 = d6, or d2 = d4 =
+// d6 = 0, one of vb, vc is <= 0 as computed and the edge a b is taken. w is NaN where a corner is not
 // finite, and d2 too: every comparison with its bounds fails, and the triangle is left to the exact step.
 #pragma once
 
@@ -118,8 +123,10 @@ __device__ __forceinline__ void tri_frame(f3 fa, f3 fb, f3 fc, float4* out) {
     e2x = cx * r;
     e2y = cy * r;
   }
-  const float wide = static_cast<float>((flat ? 512.0 : 256.0) * 5.9604644775390625e-08 * 1.0001 * ll);
-  const float f0w = l0 + l1 + l2 < 1e300 ? (flat ? -wide : wide) : __builtin_nanf("");
+  const bool equal = l0 == 0 || l1 == 0 || l2 == 0;
+  const float wide = static_cast<float>((flat && !equal ? 512.0 : 256.0) * 5.9604644775390625e-08 * 1.0001 * ll);
+  const bool unsure = flat && (equal ? l0 == 0 && l1 != 0 : true);
+  const float f0w = l0 + l1 + l2 < 1e300 ? (unsure ? -wide : wide) : __builtin_nanf("");
   // p0 is one of the float vertices: the conversion is exact
   out[0] = make_float4(static_cast<float>(p0.x), static_cast<float>(p0.y), static_cast<float>(p0.z), f0w);
   out[1] = make_float4(static_cast<float>(u.x), static_cast<float>(u.y), static_cast<float>(u.z), static_cast<float>(L));
