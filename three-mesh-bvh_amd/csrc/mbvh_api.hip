@@ -3252,7 +3252,7 @@ extern "C" int mbvh_scene_create(mbvh_ctx* ctx, const mbvh_mesh* const* meshes, 
   if ((rc = reserve_stack(ctx, std::max(max_stack_rays4, std::max(max_stack_points, max_stack_points4))))) return rc;
   // the raycast's rows, here so that the device-pointer entry points allocate nothing (without them
   // it takes one lane per ray)
-  if (ensure_buffer(ctx->contenders, (kHeavyCap * kSceneRow + kScenePool) * sizeof(uint2) + 2 * kHeavyCap * sizeof(uint32_t))) {
+  if (ensure_buffer(ctx->contenders, (kHeavyCap * kSceneRowMax + kScenePool) * sizeof(uint2) + 2 * kHeavyCap * sizeof(uint32_t))) {
     ctx->contenders = DeviceBuffer{};
     clear_error();
   }
@@ -3640,7 +3640,7 @@ int enqueue_scene(mbvh_ctx* ctx, const mbvh_scene* sc, const float* o, const flo
   a.tlas4_bigleaf = sc->d_tlas4_bigleaf;
   a.slots = sc->d_slots;
   a.contenders = static_cast<uint2*>(ctx->contenders.ptr);
-  a.contender_pool = a.contenders + kHeavyCap * kSceneRow;
+  a.contender_pool = a.contenders + kHeavyCap * kSceneRowMax;
   a.contender_pool_count = static_cast<uint32_t*>(ctx->queue.ptr) + 16;  // beside the long walks' counter's line
   a.contender_pool_cap = kScenePool;
   a.tlas_bound = sc->tlas_bound;
@@ -3752,7 +3752,7 @@ int enqueue_scene_points(mbvh_ctx* ctx, const mbvh_scene* sc, const float* point
     a.tlas4_bigleaf = sc->d_tlas4_bigleaf;
     a.point_slots = sc->d_point_slots;
     a.contenders = static_cast<uint2*>(ctx->contenders.ptr);
-    a.contender_pool = a.contenders + kHeavyCap * kSceneRow;
+    a.contender_pool = a.contenders + kHeavyCap * kSceneRowMax;
     a.contender_pool_count = static_cast<uint32_t*>(ctx->queue.ptr) + 16;
     a.contender_pool_cap = kScenePool;
     a.queue = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->queue.ptr) + kWalkQueueOffset);
@@ -3782,7 +3782,7 @@ int enqueue_scene_points(mbvh_ctx* ctx, const mbvh_scene* sc, const float* point
       SceneArgs r = a;  // the points it left
       r.heavy = nullptr;
       r.queue = a.rest_queue;
-      const uint64_t threads = launch_threads(std::min<uint64_t>(4 * a.n, kSceneRestThreads), ctx->max_threads);
+      const uint64_t threads = launch_threads(4 * a.n, ctx->max_threads);
       r.stack = stack_of(ctx, threads / 4);
       MBVH_HIP(launch_scene_closest_point4(r, threads, s));
       MBVH_HIP(launch_scene_closest_point_wide(r, kSceneWideWaves, s));

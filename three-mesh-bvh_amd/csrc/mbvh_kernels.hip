@@ -2486,8 +2486,9 @@ struct SceneCands {
 };
 constexpr uint32_t kSceneBatch = 64;
 // Points the FP32 walk leaves for the size of their lists get a wave each up to this many, four lanes in
-// FP64 beyond: 40 coincident spheres of 40,000 triangles, 30,000 points 74 ms against 100, 262,144
-// points 560 ms against 467.
+// FP64 beyond: 40 coincident spheres of 40,000 triangles, 30,000 points left 74 ms against 100, 262,144
+// points 560 ms against 467; 201,000 points far from 60 / 500 instances of up to 50,000 triangles 5.5 / 4.6 ms,
+// with the line at 32,768 6.4 / 8.2.
 constexpr uint32_t kSceneRestWide = 65536;
 constexpr uint64_t kScenePointWaves = 4096;
 constexpr uint32_t kPooled = 0xFFFFFFFDu;  // a row's first word: its contenders are in the pool
@@ -4096,6 +4097,18 @@ constexpr int kPointCand = 4;       // listed candidates per lane, besides the o
 constexpr int kPointWideCand = 12;  // the same where a point has a wave
 constexpr float kTiny = 1e-30f;
 
+// Appends v to a list for the lanes of the wave that ask for it, with one atomic: a counter takes one every 11
+// ns (262,144 points left one by one: 2.9 ms).
+__device__ __forceinline__ void wave_append(uint32_t* list, uint32_t* count, bool mine, uint32_t v) {
+  const uint64_t m = __ballot(mine);
+  if (m == 0) return;
+  const uint32_t lane = threadIdx.x & 63u, first = static_cast<uint32_t>(__builtin_ctzll(m));
+  uint32_t at = 0;
+  if (lane == first) at = atomicAdd(count, static_cast<uint32_t>(__popcll(m)));
+  at = __builtin_amdgcn_readlane(at, first);
+  if (mine) list[at + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)))] = v;
+}
+
 __device__ __forceinline__ float wave_min_f(float v) {
   for (int m = 1; m < 64; m <<= 1) v = fminf(v, __shfl_xor(v, m, 64));
   return v;
@@ -4214,9 +4227,9 @@ struct ScenePointLane {
 template <typename Share>
 __device__ __forceinline__ bool scene_point_row(const SceneArgs& A, uint64_t v, uint32_t total, bool first, Share share,
                                                 uint2*& to) {
-  uint2* const row = A.contenders + static_cast<uint64_t>(kSceneRow) * v;
+  uint2* const row = A.contenders + static_cast<uint64_t>(kPointRow) * v;
   to = row;
-  if (total > kSceneRow) {
+  if (total > kPointRow) {
     uint32_t at = 0;
     if (first) at = atomicAdd(A.contender_pool_count, total);
     at = share(at);
@@ -4226,7 +4239,7 @@ __device__ __forceinline__ bool scene_point_row(const SceneArgs& A, uint64_t v, 
       row[0] = make_uint2(kPooled, at);
       row[1] = make_uint2(total, 0u);
     }
-  } else if (first && total < kSceneRow) {
+  } else if (first && total < kPointRow) {
     row[total] = make_uint2(kNoHit, 0u);
   }
   return true;
@@ -4358,13 +4371,10 @@ __global__ __launch_bounds__(kBlock, 6) void k_scene_point_walk4(SceneArgs A) {
       left = !scene_point_row(A, v, h0 + h1 + h2 + h3, q4 == 0, [](uint32_t at) { return quad_bcast<0>(at); }, to);
       if (!left) L.write(to + (q4 == 0 ? 0u : (q4 == 1 ? h0 : (q4 == 2 ? h0 + h1 : h0 + h1 + h2))));
     }
-    if ((heavy || left) && q4 == 0) {
-      A.contenders[static_cast<uint64_t>(kSceneRow) * v] = make_uint2(kOverflow, 0u);  // not for the resolution yet
-      if (heavy)
-        A.heavy[atomicAdd(A.heavy_count, 1u)] = v;
-      else
-        A.rest[atomicAdd(A.rest_count, 1u)] = v;
-    }
+    if ((heavy || left) && q4 == 0)
+      A.contenders[static_cast<uint64_t>(kPointRow) * v] = make_uint2(kOverflow, 0u);  // not for the resolution yet
+    wave_append(A.heavy, A.heavy_count, heavy && q4 == 0, v);
+    wave_append(A.rest, A.rest_count, left && q4 == 0, v);
   }
 }
 
@@ -4489,7 +4499,7 @@ __global__ __launch_bounds__(64) void k_scene_point_wide(SceneArgs A) {
 __global__ __launch_bounds__(kBlock) void k_scene_point_resolve(SceneArgs A) {
   const uint64_t v = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (v >= A.n) return;
-  const uint2* c = A.contenders + kSceneRow * v;
+  const uint2* c = A.contenders + kPointRow * v;
   const uint2 c0 = c[0];
   if (c0.x == kOverflow) return;  // left to the FP64 walk
   uint32_t count = 0;
@@ -4497,7 +4507,7 @@ __global__ __launch_bounds__(kBlock) void k_scene_point_resolve(SceneArgs A) {
     count = c[1].x;
     c = A.contender_pool + c0.y;
   } else {
-    while (count < kSceneRow && c[count].x != kNoHit) count++;
+    while (count < kPointRow && c[count].x != kNoHit) count++;
   }
   const uint64_t i = A.order ? A.order[v] : v;
   const D3 p = d3(A.origins[3 * i], A.origins[3 * i + 1], A.origins[3 * i + 2]);
