@@ -72,6 +72,42 @@ def test_zero_direction_components(ctx, meshes, kind):
     assert (_check(ctx, ms, w)["face"][rows] != M.NO_HIT).any()
 
 
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("side", [M.FRONT_SIDE, M.DOUBLE_SIDE])
+def test_rays_along_box_planes(ctx, two, side):
+    """Rays parallel to one or two axes from whole coordinates, where the boxes of unrotated instances begin as
+    well: the reference's split-plane shortcut then skips children that may hold the nearer hit."""
+    rng = np.random.default_rng(27)
+    at = rng.integers(-6, 7, (400, 3)).astype(float)
+    axis = rng.integers(0, 3, 400)
+    quads = np.repeat(at[:, None], 4, 1)
+    u, v = np.eye(3)[(axis + 1) % 3], np.eye(3)[(axis + 2) % 3]
+    quads[:, 1] += u
+    quads[:, 2] += u + v
+    quads[:, 3] += v
+    f = np.arange(400)[:, None] * 4
+    g, idx, tree = build_mesh(G.Geometry(quads.reshape(-1, 3).astype(np.float32),
+                                         np.concatenate([f, f + 1, f + 2, f, f + 2, f + 3], 1).reshape(-1).astype(np.uint32)),
+                              leaf=1)
+    ms = [ctx.upload(tree, g.positions, idx)]
+    w = W.scene_rays([g], 4, 4000, seed=28)
+    for k in range(4):
+        m = np.eye(4)
+        m[:3, 3] = rng.integers(-9, 10, 3)
+        w.matrix_world[k] = m.T.reshape(-1)
+        w.matrix_world_inverse[k] = np.linalg.inv(m).T.reshape(-1)
+    d = rng.choice([-1.0, 1.0], (4000, 3)) * (1.0 if two else rng.uniform(0.2, 1.0, (4000, 3)))
+    zero = rng.integers(0, 3, 4000)
+    d[np.arange(4000), zero] = np.where(rng.random(4000) < 0.5, 0.0, -0.0)
+    if two:
+        d[np.arange(4000), (zero + 1) % 3] = 0.0
+    w.directions[:] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    w.origins[:] = rng.integers(-12, 13, (4000, 3))
+    ref = _check(ctx, ms, w, side=side)
+    assert (ref["face"] != M.NO_HIT).sum() > 500
+    ms[0].free()
+
+
 @pytest.mark.parametrize("kind", ["shifted", "scaled", "projective", "sheared"])
 def test_any_inverse(ctx, meshes, kind):
     geos, ms = meshes

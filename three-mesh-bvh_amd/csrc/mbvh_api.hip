@@ -2909,8 +2909,6 @@ constexpr uint32_t kSceneHeavyBudget = 512;
 constexpr uint32_t kScenePointBudget = 100;
 constexpr uint64_t kScenePointMin = 200000;
 constexpr uint32_t kSceneWideWaves = 2048;
-// Threads over the rays the four-lane raycast leaves (usually none).
-constexpr uint64_t kSceneRestThreads = 1u << 17;
 
 struct mbvh_scene {
   uint32_t magic = 0x4E454353u;  // "SCEN"
@@ -3660,7 +3658,7 @@ int enqueue_scene(mbvh_ctx* ctx, const mbvh_scene* sc, const float* o, const flo
     const uint64_t quads = launch_threads(4 * a.n, ctx->max_threads) / 4;
     a.stack = stack_of(ctx, quads);
     MBVH_HIP(launch_scene_raycast_first4(a, quads, s));
-    const uint64_t threads = launch_threads(std::min<uint64_t>(a.n, kSceneRestThreads), ctx->max_threads);
+    const uint64_t threads = launch_threads(a.n, ctx->max_threads);
     a.stack = stack_of(ctx, threads);
     MBVH_HIP(launch_scene_raycast_first(a, threads, s));
   }

@@ -2447,9 +2447,11 @@ __global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
 // end is dropped, one wholly before theirs replaces them, otherwise its candidates join them.
 // k_scene_ray_resolve settles each ray's contenders (nearly always one triangle) as the one-lane kernel does:
 // per instance the exact first hit with the reference's tie rule, then the least world distance,
-// equal ones to the lower instance. Rays with a zero direction component, in the world or in an
-// instance they reach, and rays with more contenders than a row holds go to the one-lane kernel
-// (A.heavy lists them).
+// equal ones to the lower instance. Rays with more contenders than a quad holds go to the one-lane
+// kernel (A.heavy lists them), and so do rays whose hit the reference's split-plane shortcut may change:
+// where the direction is zero along a node's split axis, it skips the far (right) child once the near one
+// has had a hit and the far box begins at or past the origin. A box that begins past it the ray does not
+// enter, so a nearest hit that is skipped is a contender that begins at the origin on that axis.
 //
 // What bounds it: vector issue (1.5 of 2.0 ms for 512 instances and 2^20 rays from outside; about 20
 // node, 4 triangle and 5 switch steps per ray, half the lanes busy) at four waves per SIMD (126
@@ -2497,13 +2499,17 @@ constexpr uint64_t kScenePointWaves = 4096;
 constexpr uint32_t kPooled = 0xFFFFFFFDu;  // a row's first word: its contenders are in the pool
 constexpr uint32_t kContend = 16;         // contenders a quad holds
 
+constexpr float kParallelRcp = 1.2676506002282294e30f;  // 2^100, scene_box4's reciprocal of zero
 // ray_box4 for the scene's quads: the reciprocals by the hardware's 1-ulp instruction. That is u more
-// relative error than a division on both plane products, 6 u S of the widening's 8 u S. False: a zero
-// direction component or constants that are not finite (literal_ray).
+// relative error than a division on both plane products, 6 u S of the widening's 8 u S. A zero direction
+// component has the reciprocal 2^100: the widening then takes in every box whose slab holds the origin
+// (and those within 8 u of the coordinates of it) for all t, and leaves the others. False: no direction, or
+// constants that are not finite.
+__device__ __forceinline__ float scene_rcp(float d) { return d == 0.0f ? kParallelRcp : rcp_approx(d); }
 __device__ __forceinline__ bool scene_box4(f3 o, f3 d, float coord_max, RayBox4& r) {
-  r.ix = rcp_approx(d.x);
-  r.iy = rcp_approx(d.y);
-  r.iz = rcp_approx(d.z);
+  r.ix = scene_rcp(d.x);
+  r.iy = scene_rcp(d.y);
+  r.iz = scene_rcp(d.z);
   const float ox = -o.x * r.ix, oy = -o.y * r.iy, oz = -o.z * r.iz;
   const float ex = 8.0f * kU * ((coord_max + fabsf(o.x)) * fabsf(r.ix));
   const float ey = 8.0f * kU * ((coord_max + fabsf(o.y)) * fabsf(r.iy));
@@ -2519,7 +2525,8 @@ __device__ __forceinline__ bool scene_box4(f3 o, f3 d, float coord_max, RayBox4&
   r.sz = r.iz >= 0.0f;
   // a sub-2^-126 reciprocal is flushed to zero: |d| that large is left to the one-lane kernel too
   const float big = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
-  return fabsf(r.ix) + fabsf(r.iy) + fabsf(r.iz) + fabsf(ox) + fabsf(oy) + fabsf(oz) + ex + ey + ez < kInf && big < 1e30f;
+  return fabsf(r.ix) + fabsf(r.iy) + fabsf(r.iz) + fabsf(ox) + fabsf(oy) + fabsf(oz) + ex + ey + ez < kInf && big < 1e30f &&
+         big > 0.0f;
 }
 
 // The terms of a ray's world distance in an instance's frame: t * along within off + t * grow. From the
@@ -2893,7 +2900,17 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
   }
 }
 
-// The contenders of the rays settled, one lane per ray.
+// Whether the triangle begins at the ray's origin (within twice the box widening) on an axis along which the
+// direction is zero.
+__device__ __forceinline__ bool begins_at_origin(f3 o, f3 d, float coord_max, const Tri& t) {
+  auto at = [&](float dk, float ok, float a, float b, float c) {
+    return dk == 0.0f && fabsf(fminf(fminf(a, b), c) - ok) <= 16.0f * kU * (coord_max + fabsf(ok));
+  };
+  return at(d.x, o.x, t.p0.x, t.p1.x, t.p2.x) || at(d.y, o.y, t.p0.y, t.p1.y, t.p2.y) || at(d.z, o.z, t.p0.z, t.p1.z, t.p2.z);
+}
+
+// The contenders of the rays settled, one lane per ray; a ray with one on which the split-plane shortcut may act is
+// left to the one-lane kernel.
 __global__ __launch_bounds__(kBlock) void k_scene_ray_resolve(SceneArgs A) {
   const uint64_t ray = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (ray >= A.n) return;
@@ -2926,6 +2943,10 @@ __global__ __launch_bounds__(kBlock) void k_scene_ray_resolve(SceneArgs A) {
       if (c[i].y != inst) continue;
       const uint32_t slot = c[i].x;
       const Tri tr = load_tri(M.tris, slot);
+      if (begins_at_origin(o, d, *M.coord_max, tr)) {
+        A.heavy[atomicAdd(A.heavy_count, 1u)] = static_cast<uint32_t>(ray);
+        return;
+      }
       ff t;
       if (!hit_exact<false>(o, d, z, z, tr.a(), tr.b(), tr.c(), A.side_mask ? A.side_mask : tr.mask(), win, t)) continue;
       bool take = w == kNoHit;
