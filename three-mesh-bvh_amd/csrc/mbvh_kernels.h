@@ -300,6 +300,11 @@ struct SceneArgs {
   uint2* contender_pool;           // rows of the rays with more
   uint32_t* contender_pool_count;
   uint32_t contender_pool_cap;
+  // raycast, four lanes: set, the launch first decides by the rays' coherence whether the one-lane kernel takes
+  // them all (*one_lane; a.n >= 4096): the spread up to which 64 rays are coherent, 1 / the scene's size
+  uint32_t* one_lane;
+  float coherent;
+  float per_size;
   const float* world;              // 16 floats per instance (local -> world, column-major)
   const float* inverse;            // 16 floats per instance (world -> local)
   // closest point's box bounds in the instance frame: 16 floats per instance, the float rounding of
@@ -336,7 +341,7 @@ struct SceneArgs {
   uint32_t* more_count;
   uint32_t* rest_queue;
 };
-// One lane per ray, over a.heavy (*a.heavy_count rays) or, when it is NULL, every ray.
+// One lane per ray, over a.heavy (*a.heavy_count rays) or, when it is NULL or *a.one_lane is set, every ray.
 hipError_t launch_scene_raycast_first(const SceneArgs& a, uint64_t threads, hipStream_t s);
 // Four lanes per ray (quads: rays traced at once, a multiple of 64; a.n < 2^32) and the resolution of
 // their contenders; the rays it leaves are listed in a.heavy, which must hold a.n entries.

@@ -2326,7 +2326,8 @@ __device__ __forceinline__ bool box_entry(f3 o, f3 inv, const float* b, float ne
   return tmin <= tmax && tmax >= near_dist;
 }
 
-// One lane per ray, for the rays the four-lane kernel left (A.heavy lists them; NULL: every ray). The
+// One lane per ray, for the rays the four-lane kernel left (A.heavy lists them) or, where that is NULL or
+// *A.one_lane says so, every ray. The
 // TLAS (reference node format over the instances' world boxes, expanded
 // outward when built) is walked near child first and pruned by the best world distance so far
 // (with a 2^-16 relative margin: box distances and hit distances round differently); each
@@ -2334,8 +2335,10 @@ __device__ __forceinline__ bool box_entry(f3 o, f3 inv, const float* b, float ne
 // per-instance launch does (near / far scaled by the instance, hit point and distance back in world
 // space), so every instance's hit is that launch's hit. The closest world distance wins; equal
 // distances keep the lowest instance index, the order a stable sort of the reference's
-// per-instance hits (acceleratedBatchedMeshRaycast) gives.
-__global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
+// per-instance hits (acceleratedBatchedMeshRaycast) gives. Three workgroups per compute unit, as many as its
+// LDS allows: left to itself the compiler takes 169 registers, one too many for the third (2^20 rays into one
+// instance 1.02 -> 1.36 ms).
+__global__ __launch_bounds__(kBlock, 3) void k_scene_raycast_first(SceneArgs A) {
   __shared__ uint2 lds_stack[8 * kBlock];
   __shared__ uint32_t tstack[kSceneStack * kBlock];
   const uint32_t tid = threadIdx.x;
@@ -2349,9 +2352,10 @@ __global__ __launch_bounds__(kBlock) void k_scene_raycast_first(SceneArgs A) {
   st.capacity = 8 + static_cast<int>(A.stack.ovf_entries);
   const float qnan = __int_as_float(0x7fc00000);
   const float margin = 1.0f + 1.0f / 65536.0f;
-  const uint64_t count = A.heavy ? static_cast<uint64_t>(*A.heavy_count) : A.n;
+  const bool all = !A.heavy || (A.one_lane && *A.one_lane);
+  const uint64_t count = all ? A.n : static_cast<uint64_t>(*A.heavy_count);
   for (uint64_t k = gtid; k < count; k += static_cast<uint64_t>(gridDim.x) * kBlock) {
-    const uint64_t ray = A.heavy ? A.heavy[k] : k;
+    const uint64_t ray = all ? k : A.heavy[k];
     const f3 ow = mk(A.origins[3 * ray], A.origins[3 * ray + 1], A.origins[3 * ray + 2]);
     const f3 dw = mk(A.directions[3 * ray], A.directions[3 * ray + 1], A.directions[3 * ray + 2]);
     const f3 iw = mk(1.0f / dw.x, 1.0f / dw.y, 1.0f / dw.z);
@@ -2583,6 +2587,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_raycast_first4(SceneArgs A)
   __shared__ uint2 contend[kContend * (kBlock / 4)];  // (slot, instance)
   __shared__ float4 wbox[2 * (kBlock / 4)];
   __shared__ float wbox_hz[kBlock / 4];
+  if (A.one_lane && *A.one_lane) return;
   const uint32_t lane = threadIdx.x, wl = lane & 63u, q4 = lane & 3u, qid = lane >> 2;
   SceneStack st;
   st.lds = qstack;
@@ -2913,7 +2918,7 @@ __device__ __forceinline__ bool begins_at_origin(f3 o, f3 d, float coord_max, co
 // left to the one-lane kernel.
 __global__ __launch_bounds__(kBlock) void k_scene_ray_resolve(SceneArgs A) {
   const uint64_t ray = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (ray >= A.n) return;
+  if (ray >= A.n || (A.one_lane && *A.one_lane)) return;
   const uint2* c = A.contenders + kSceneRow * ray;
   const uint2 c0 = c[0];
   if (c0.x == kOverflow) return;  // left to the one-lane kernel
@@ -4828,15 +4833,37 @@ hipError_t launch_batch_raycast_first(const BatchArgs& a, uint32_t stack_lds, ui
   return hipGetLastError();
 }
 
-__global__ void k_scene_reset(uint32_t* queue, uint32_t* count, uint32_t* pool_count) {
-  if (threadIdx.x < kWalkQueues) queue[32 * threadIdx.x] = 0u;
-  if (threadIdx.x == 0) *count = *pool_count = 0u;
+// Clears the counters of a four-lane raycast and, where A.one_lane is set, decides whether one lane per ray takes
+// the call: where most of the samples, 64 consecutive rays each, stay within A.coherent (their directions'
+// spread and their origins' over the scene's size, added). Such rays share nodes within a wave of 64, which four
+// lanes per ray make four times the steps of.
+__global__ __launch_bounds__(1024) void k_scene_reset(SceneArgs A) {
+  if (threadIdx.x < kWalkQueues) A.queue[32 * threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *A.heavy_count = *A.contender_pool_count = 0u;
+  if (!A.one_lane) return;
+  __shared__ uint32_t close;
+  if (threadIdx.x == 0) close = 0u;
+  __syncthreads();
+  constexpr uint32_t kSamples = 64;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t tiles = A.n / 64;  // A.n is 64 kSamples or more
+  for (uint32_t k = threadIdx.x >> 6; k < kSamples; k += 16) {
+    const uint64_t ray = tiles * k / kSamples * 64 + lane;
+    const f3 o = load3(A.origins, ray), d = load3(A.directions, ray);
+    const float per = __builtin_amdgcn_rsqf(dot(d, d));
+    const f3 n = mk(d.x * per, d.y * per, d.z * per);
+    const f3 dn = sub(n, mk(__shfl(n.x, 0, 64), __shfl(n.y, 0, 64), __shfl(n.z, 0, 64)));
+    const f3 dp = sub(o, mk(__shfl(o.x, 0, 64), __shfl(o.y, 0, 64), __shfl(o.z, 0, 64)));
+    const float spread = __builtin_amdgcn_sqrtf(dot(dn, dn)) + __builtin_amdgcn_sqrtf(dot(dp, dp)) * A.per_size;
+    if (__ballot(spread <= A.coherent) == ~0ull && lane == 0) atomicAdd(&close, 1u);  // NaN: not close
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *A.one_lane = 2 * close > kSamples ? 1u : 0u;
 }
 
 hipError_t launch_scene_raycast_first4(const SceneArgs& a, uint64_t quads, hipStream_t s) {
   if (a.n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scene_reset, dim3(1), dim3(64), 0, s, a.queue, a.heavy_count,
-                     a.contender_pool_count);
+  hipLaunchKernelGGL(k_scene_reset, dim3(1), dim3(a.one_lane ? 1024 : 64), 0, s, a);
   hipLaunchKernelGGL(k_scene_raycast_first4, dim3(static_cast<uint32_t>(quads / (kBlock / 4))), dim3(kBlock), 0, s, a);
   hipLaunchKernelGGL(k_scene_ray_resolve, dim3(static_cast<uint32_t>((a.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a);
   return hipGetLastError();
