@@ -1705,7 +1705,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_closest_point4(ClosestPointArgs A
             // every candidate that may tie stays listed: ties go to the reference's first
             const bool sure = !signbit_of(f0.w);
             if (sure) Ul = fminf(Ul, d2 + e2);
-            if (!sure | (cl.n == kCand)) {  // both rare: one branch
+            if (__builtin_expect(!sure | (cl.n == kCand), 0)) {
               if (!sure) Ul = fminf(Ul, exact_bound<kLo>(q, ql, M.tris, s));
               if (cl.n == kCand && !cl.compact(Ul)) {
                 const Winner r = resolve_point<kLo, true>(cl, Ul, q, ql, M.tris, T);
