@@ -162,3 +162,50 @@ def test_segments(setup, corners):
     np.testing.assert_allclose(got["distance"], np.tile(d.min(1), LEAST // 2000), rtol=1e-6)
     sc.free()
     mesh.free()
+
+
+def _roots(g, parts):
+    """The geometry's triangles in `parts` ranges, a root each."""
+    edges = np.linspace(0, g.index.size // 3, parts + 1).astype(int)
+    return [(int(a), int(b - a)) for a, b in zip(edges[:-1], edges[1:])]
+
+
+def test_several_roots(setup):
+    """Instances of a mesh of four roots among others."""
+    ctx, meshes = setup
+    g = G.torus_knot(0.8, 0.25, 90, 9, 2, 3).ensure_index()
+    g, idx, tree = build_mesh(g, ranges=_roots(g, 4))
+    assert len(tree.roots) == 4
+    mesh = ctx.upload(tree, g.positions, idx)
+    rng = np.random.default_rng(10)
+    check((ctx, [mesh, meshes[0]]), matrices(9, rng), np.arange(9) % 2, rng.uniform(-7, 7, size=(3000, 3)))
+    mesh.free()
+
+
+def test_second_part(setup):
+    """More points than a launch takes, in the caller's visit order (outputs in place) and without one (the
+    second part's buffers moved)."""
+    import torch
+
+    ctx, meshes = setup
+    rng = np.random.default_rng(11)
+    m = matrices(5, rng)
+    world = np.ascontiguousarray(m.transpose(0, 2, 1).reshape(-1, 16), dtype=np.float32)
+    inverse = np.linalg.inv(world.reshape(-1, 4, 4).astype(np.float64)).reshape(-1, 16).astype(np.float32)
+    sc = ctx.scene(meshes, world, inverse, np.arange(5, dtype=np.uint32) % 3)
+    n = (1 << 20) + 4321
+    q = rng.uniform(-8, 8, (n, 3)).astype(np.float32)
+    ctx.set_point_lanes(1)
+    ref = sc.closest_point(q)
+    ctx.set_point_lanes(0)
+    points = torch.as_tensor(q, device="cuda")
+    order = torch.as_tensor(rng.permutation(n).astype(np.uint32).view(np.int32), device="cuda")
+    for visit in (0, order.data_ptr()):
+        out = {k: torch.full((n, 3) if k in ("point", "barycoord") else (n,), -7, dtype=torch.int32, device="cuda")
+               for k in ("face", "instance", "distance", "point", "barycoord")}
+        torch.cuda.synchronize()
+        sc.closest_point_d(points.data_ptr(), n, *[out[k].data_ptr() for k in out], order_ptr=visit)
+        ctx.synchronize()
+        for k in ref:
+            np.testing.assert_array_equal(out[k].cpu().numpy(), ref[k].view(np.int32), err_msg=k)
+    sc.free()

@@ -8,6 +8,7 @@ import mbvh_amd as M
 from mbvh_amd import geometry as G, workloads as W
 from helpers import build_mesh
 from test_gpu_scene import GEOMS, _pairwise, _same
+from test_gpu_scene_points import _roots
 
 pytestmark = pytest.mark.gpu
 
@@ -169,3 +170,15 @@ def test_many_rays(ctx, meshes, kind, count, n):
         w.directions[:] = (at - eye) / np.linalg.norm(at - eye, axis=1, keepdims=True)
     ref = _check(ctx, ms, w)
     assert (ref["face"] != M.NO_HIT).sum() > n // 100
+
+
+def test_several_roots(ctx, meshes):
+    """Instances of a mesh of four roots among others."""
+    geos, ms = meshes
+    g = G.torus_knot(0.8, 0.25, 90, 9, 2, 3).ensure_index()
+    g, idx, tree = build_mesh(g, ranges=_roots(g, 4))
+    assert len(tree.roots) == 4
+    mesh = ctx.upload(tree, g.positions, idx)
+    ref = _check(ctx, [mesh, ms[0]], W.scene_rays([g, geos[0]], 9, 2000, seed=30))
+    assert (ref["face"] != M.NO_HIT).any()
+    mesh.free()
