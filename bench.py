@@ -1031,10 +1031,11 @@ def main():
                 "tris_per_query": round(tris, 2), "kernel_ms": round(kern_ms, 4),
                 "kernel": "k_closest_point_packet"}
         if valu:
-            # the measured limiter: VALU issue (HBM traffic is a small fraction of the algorithmic
-            # bytes: node and triangle reads hit in the caches)
+            # VALU issue of the committed profile of this kernel; where it is the smaller part of the call, the
+            # packets wait for the scalar loads of the next node or triangle frame (HBM traffic is a small
+            # fraction of the algorithmic bytes: node and frame reads hit in the caches)
             valu_ms = valu * 4 / (SIMDS * CLOCK_GHZ * 1e9) * 1e3
-            roof["limiter"] = "VALU issue"
+            roof["limiter"] = "VALU issue" if valu_ms > 0.6 * kern_ms else "latency of scalar loads"
             roof["valu_insts_per_launch"] = round(valu)
             roof["valu_issue_ms"] = round(valu_ms, 3)
             roof["valu_issue_frac"] = round(valu_ms / kern_ms, 3)
