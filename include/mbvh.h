@@ -14,10 +14,11 @@
  *     hipStream_t, or NULL for the context's own stream). They allocate nothing and never
  *     synchronise, so a caller may capture them in a HIP graph. The other query entry points
  *     take HOST pointers and are synchronous.
- *   - All query kernels of one context share that context's work-queue counter and traversal
- *     stack overflow region. The "_d" calls of one context must therefore be serialised: issue
+ *   - All query kernels of one context share that context's work queues and their counters, the lists of
+ *     queries handed from one kernel of a call to the next, the scene queries' candidate rows and the
+ *     traversal stack overflow region. The "_d" calls of one context must therefore be serialised: issue
  *     them on one stream (or order the streams with events). Two "_d" calls of one context that
- *     run at the same time on different streams overwrite each other's spilled stack entries.
+ *     run at the same time on different streams overwrite each other's entries and give wrong answers.
  *     Use one context per stream for concurrent queries.
  *   - Vectors are packed float triples (x, y, z) per element.
  *   - A miss is reported as face index MBVH_NO_HIT and distance +Infinity.
@@ -171,7 +172,9 @@ int mbvh_build_gpu_d(mbvh_ctx* ctx, const float* positions, uint64_t vertex_coun
 /*
  * Uploads one MeshBVH (its serialized form, MeshBVH.serialize src/core/MeshBVH.js:112-145:
  * roots, index, indirectBuffer) plus its float32 positions to HBM, once. The library derives its
- * traversal layout from those buffers on upload; later queries read only device memory.
+ * traversal layout from those buffers on upload; later queries read only device memory. Beside the
+ * tree a mesh takes 140 bytes per triangle there: corners 48, vertex ids 12, and 80 for the frame the
+ * closest-point queries measure by, which a refit rewrites.
  * index may be NULL only when an indirect buffer is given (non-indexed indirect build).
  */
 int mbvh_mesh_upload(mbvh_ctx* ctx, const void* const* roots, const uint64_t* root_bytes,
@@ -554,7 +557,8 @@ int mbvh_mesh_import_textures(mbvh_ctx* ctx, const float* bvh_bounds, const uint
  * rejected with MBVH_ERR_BAD_ARGS. matrix_world_inverse is used as given to bring rays into each
  * instance's frame (as raycastObject3D inverts matrixWorld itself); the closest point's pruning
  * bounds never rely on it: the scene computes its own inverse in double and uses world boxes for an
- * instance whose inverse fails a residual check.
+ * instance whose inverse fails a residual check. The first scene of a context allocates 88 MiB of
+ * candidate rows and lists that all its scenes' queries share (without them the queries are slower).
  */
 int mbvh_scene_create(mbvh_ctx* ctx, const mbvh_mesh* const* meshes, uint32_t n_meshes, const float* matrix_world,
                       const float* matrix_world_inverse, const uint32_t* instance_geometry, const uint8_t* visible,
@@ -582,9 +586,10 @@ int mbvh_scene_raycast_first_d(mbvh_ctx* ctx, const mbvh_scene* scene, const flo
  * barycoord (NULL outputs other than face_index are skipped). Host-pointer form (synchronous; it
  * orders the points spatially itself) and device-pointer form (enqueues on `stream`; `order`: NULL or
  * a visit order of the n points such as mbvh_order_points_d writes, which lets the lanes of a wave
- * share instances and tree paths; face 0xFFFFFFFE marks a traversal stack overflow). Points whose
- * walks are long finish in a pass of one wave each, through a list the context allocates once: in
- * calls of up to 2^20 points.
+ * share instances and tree paths; face 0xFFFFFFFE marks a traversal stack overflow). From 200,000 points
+ * on, and where every matrix_world is a similarity (to 2^-13), the walk is in FP32 and its candidates are
+ * settled in double: the same answers. Points whose walks are long finish in a pass of one wave each,
+ * through lists the context allocates with its first scene; without that walk, in calls of up to 2^20 points.
  */
 int mbvh_scene_closest_point(mbvh_ctx* ctx, const mbvh_scene* scene, const float* points, uint64_t n,
                              uint32_t* face_index, uint32_t* instance, float* distance, float* point,

@@ -56,7 +56,7 @@ struct mbvh_ctx {
   DeviceBuffer order;           // host-API query order
   DeviceBuffer order_ws;        // host-API ordering workspace
   DeviceBuffer heavy;           // queries left to a wave each (kHeavyCap entries, allocated with the context)
-  DeviceBuffer contenders;      // scene raycast: kSceneRow per ray of a launch (allocated with the first scene)
+  DeviceBuffer contenders;      // scene queries: a row per query of a launch, the pool, the points left (allocated with the first scene)
   DeviceBuffer hits[5];         // host-API all-hits results: offsets, face, dist, point, bary
   DeviceBuffer grad[11];        // host-API backward staging
   DeviceBuffer grad_ws;         // host-API backward workspace
@@ -3770,10 +3770,11 @@ int enqueue_scene_points(mbvh_ctx* ctx, const mbvh_scene* sc, const float* point
   a.out_point = point;
   a.out_bary = bary;
   a.order = order;  // a spatial order lets the lanes of a wave share instances and tree paths
-  // the FP32 walk where every instance is placed by a similarity (2^20 points, 512 instances: 4.3 ms
-  // against 9.7), its lists, stacks and long walks have their room, and the points fill the chip: its
-  // steps are cheaper but not shorter, and its launches one after another (250,000 points on five scenes
-  // of 8 to 600 instances 1.03 to 2.1 times as fast, 40,000 points 0.74 to 1.8, 6,000 0.75 to 1.4)
+  // the FP32 walk where every instance is placed by a similarity (2^20 points, 512 instances: 3.1 ms
+  // against 9.4), its lists, stacks and long walks have their room, and the points fill the chip: its
+  // steps are cheaper but not shorter, and its launches one after another (201,000 points on scenes of 1 to
+  // 1,000 instances 1.4 to 3.6 times as fast; measured with 64 points taken at a time, 40,000 points on five
+  // scenes 0.74 to 1.8, 6,000 0.75 to 1.4)
   if (quads && n >= kScenePointMin && sc->similar && sc->wide_ok && ctx->heavy.ptr && ctx->contenders.ptr &&
       sc->max_stack_rays4 <= kMinLdsStack + ctx->stack_ovf_entries) {
     a.tlas4 = sc->d_tlas4;

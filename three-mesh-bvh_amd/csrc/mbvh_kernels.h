@@ -271,10 +271,10 @@ constexpr uint32_t kSceneRow = 4;       // contenders of a ray before it takes a
 // against 1.8 ms).
 constexpr uint32_t kPointRow = 6;
 constexpr uint32_t kSceneRowMax = kPointRow;
-constexpr uint32_t kScenePool = 1u << 22;  // pool entries per launch; when they are gone, the one-lane kernel
+constexpr uint32_t kScenePool = 1u << 22;  // pool entries per launch; when they are gone, the kernels of last resort
 constexpr uint32_t kSceneSlotRows = 8;  // uint4 per top-level slot
-// Scene: closest first hit over instances, one launch (TLAS over the instances' world boxes).
 constexpr uint32_t kScenePointRows = 10;
+// Scene queries over instances (TLAS over the instances' world boxes).
 struct SceneArgs {
   const MeshView* meshes;
   uint32_t n_meshes;

@@ -2457,10 +2457,10 @@ __global__ __launch_bounds__(kBlock, 3) void k_scene_raycast_first(SceneArgs A) 
 // has had a hit and the far box begins at or past the origin. A box that begins past it the ray does not
 // enter, so a nearest hit that is skipped is a contender that begins at the origin on that axis.
 //
-// What bounds it: vector issue (1.5 of 2.0 ms for 512 instances and 2^20 rays from outside; about 20
-// node, 4 triangle and 5 switch steps per ray, half the lanes busy) at four waves per SIMD (126
+// What bounds it: vector issue (1.5 of 1.9 ms for 512 instances and 2^20 rays from outside; about 20
+// node, 4 triangle and 5 switch steps per ray, half the lanes busy) at four waves per SIMD (127
 // registers; 96 spill and are slower). One lane per ray with each instance's walk nested in the top
-// level's and settled exactly on the way kept 3% of the lanes busy: 7.9 -> 2.1 ms. On the way: popping
+// level's and settled exactly on the way kept 3% of the lanes busy: 7.9 -> 2.0 ms. On the way: popping
 // one entry per step instead of looping to the next live one, no exact step in this kernel (each in a
 // quarter of its lanes), instance records in one load, each step in a loop of its own (a third fewer
 // instructions, the rest being copies of the walk's state).
@@ -4115,12 +4115,13 @@ __global__ __launch_bounds__(kBlock, 4) void k_scene_closest_point4(SceneArgs A)
 // distance, one of them in registers (the packets' rule). A point past the step budget goes to a wave of
 // its own (A.heavy, the kernel after this), one with more candidates than the lists hold to A.rest.
 //
-// What bounds it: latency and the vector-memory unit, at five waves per SIMD (512 instances of up to
+// What bounds it: latency and the vector-memory unit, at six waves per SIMD (512 instances of up to
 // 50,000 triangles, 2^20 points in Morton order: 7 top-level and 23 tree nodes, 113 triangles in 16
-// leaves per point, a wave's longest point 1.8 times that; 1.7 of 3.6 ms is vector issue). The kernel it
+// leaves per point, a wave's longest point 1.8 times that; 1.8 of 2.4 ms is vector issue). The kernel it
 // replaces there measured in FP64 as it walked the binary top level and each instance in a nest of
 // loops, with 128 registers and spills: 8.4 ms. The budget keeps the longest points from
-// outlasting the launch: 4.4 ms at 256 steps, 3.5 at 100, 3.2 at 64 (where the wave kernel takes 1.4 ms).
+// outlasting the launch (with 64 points taken at a time 4.4 ms at 256 steps, 3.5 at 100, 3.2 at 64, where the
+// wave kernel takes 1.4 ms).
 // ------------------------------------------------------------------------------------------
 constexpr int kPointCand = 4;       // listed candidates per lane, besides the one in registers
 constexpr int kPointWideCand = 12;  // the same where a point has a wave
@@ -4415,7 +4416,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_scene_point_walk4(SceneArgs A) {
 // of A.rest (A.more_count of them).
 //
 // What bounds it: the serial rounds of a point (load, reduce, push), eight waves to a compute unit:
-// 0.3 ms for some 5,000 points; one triangle per lane in turn, in FP64, took 0.8 ms for a fifth of them.
+// 0.34 ms for some 5,000 points; one triangle per lane in turn, in FP64, took 0.8 ms for a fifth of them.
 // ------------------------------------------------------------------------------------------
 constexpr uint32_t kPointFrontier = 1024;  // at most 48 entries per level of the tree and 64
 constexpr uint32_t kPointTop = 80;         // the top level's stack: three entries for each of 24 levels

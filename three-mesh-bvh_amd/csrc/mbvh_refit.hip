@@ -9,18 +9,19 @@
 // left : right, max: left > right ? left : right) exactly when a child changed, and then counts as
 // changed itself.
 //
-// Device form, level by level: one launch decides every leaf, then one launch per depth, deepest
-// first, decides the internal nodes of that depth from their children (decided by an earlier
-// launch on the same stream, so no fences or counters are needed). A node's box is written to the
-// device copy of the reference nodes and, where the node has one, to its place in the parent's wide
-// node; k_refit_four then copies the wide boxes into the 4-wide tree, and k_refit_tris re-gathers
-// the triangle corners (their .w words - face id, facing mask, vertex id - are kept). The
-// coordinate bound the query kernels scale their error bounds by is recomputed from the positions.
+// Device form, level by level: k_refit_tris re-gathers the triangle corners (their .w words - face id,
+// facing mask, vertex id - are kept) and rewrites the frames, one launch decides every leaf from them, then
+// the internal nodes are decided from their children, deepest depth first: a launch per depth of more
+// than kSmallLevel nodes (ordered by the stream, so no fences or counters are needed), one workgroup with a
+// barrier between depths for a run of smaller ones. A node's box is written to the device copy of the
+// reference nodes and, where the node has one, to its place in the parent's wide node; k_refit_four
+// then copies the wide boxes into the 4-wide tree. The coordinate bound the query kernels scale their
+// error bounds by is recomputed from the positions.
 //
 // A partial refit (nodeIndices, refit.template.js:136-172) first marks the nodes the reference's
 // traversal visits, top down, one launch per depth: every root is visited; a visited internal node
 // that is not forced visits the children in the set, or, when neither is, both, forced; a forced
-// node forces its children. The per-node word holds the marks until the bottom-up launches replace
+// node forces its children. The per-node word holds the marks until the bottom-up steps replace
 // them by the changed flag; a node not visited keeps its box and counts as unchanged. The triangle
 // corners and the coordinate bound are refreshed everywhere, as the queries read the new positions.
 #include "mbvh_kernels.h"
