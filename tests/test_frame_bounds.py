@@ -19,7 +19,8 @@ def frames(tmp_path_factory):
     if not cxx:
         pytest.skip("no host compiler")
     so = str(tmp_path_factory.mktemp("frame") / "frame_host.so")
-    subprocess.run([cxx, "-std=c++17", "-O2", "-mfma", "-ffp-contract=fast", "-w", "-shared", "-fPIC", "-I" + HERE,
+    fma = ["-mfma"] if os.path.exists("/proc/cpuinfo") and " fma " in open("/proc/cpuinfo").read() else []
+    subprocess.run([cxx, "-std=c++17", "-O2", *fma, "-ffp-contract=fast", "-w", "-shared", "-fPIC", "-I" + HERE,
                     os.path.join(HERE, "frame_host.cpp"), "-o", so], check=True)
     lib = ctypes.CDLL(so)
 
