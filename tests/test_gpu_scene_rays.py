@@ -154,17 +154,19 @@ def test_grazing_rays(ctx):
 
 
 @pytest.mark.parametrize("kind,count,n", [("random", 3, (1 << 18) + 37), ("camera", 3, (1 << 18) + 37), ("camera", 1, 140000),
-                                          ("random", 3, (1 << 20) + 1237), ("camera", 3, (1 << 20) + 300000)])
+                                          ("random", 3, (1 << 20) + 1237), ("camera", 3, (1 << 20) + 300000),
+                                          ("within", 33, (1 << 18) + 37)])
 def test_many_rays(ctx, meshes, kind, count, n):
     """Calls large enough to be sampled for coherence (a camera's rows of rays are coherent and go to one lane per
-    ray), for one instance to do without, and to be cut: a second part below and above the sampled size."""
+    ray, from within the scene also at a wider spread), for one instance to do without, and to be cut: a second
+    part below and above the sampled size."""
     geos, ms = meshes
     w = W.scene_rays(geos, count, n, seed=29)
-    if kind == "camera":
+    if kind != "random":
         k = np.arange(n) / n
         at = w.matrix_world.reshape(-1, 4, 4)[:, 3, :3]
         ctr, half = at.mean(0), np.abs(at - at.mean(0)).max() + 1.5
-        eye = ctr + half * np.array([0.5, 4.0, 0.3])
+        eye = ctr + half * np.array([0.5, 4.0, 0.3] if kind == "camera" else [0.1, 0.6, 0.1])
         at = ctr + half * np.stack([2 * (1000 * k % 1) - 1, 0 * k, 2 * k - 1], 1)
         w.origins[:] = eye
         w.directions[:] = (at - eye) / np.linalg.norm(at - eye, axis=1, keepdims=True)

@@ -2913,19 +2913,22 @@ constexpr uint32_t kSceneWideWaves = 2048;
 // Where one lane per ray is the faster scene raycast: coherent rays (a camera's, in rows) share the nodes they
 // visit within a wave, and few instances leave the four-lane walk's one loop for both levels little to gain. So in calls
 // that fill the chip with one or two instances, and up to kSceneSampled instances where a sample finds the rays
-// coherent: 64 consecutive ones within kCoherentFew (up to kSceneFew instances) or kCoherentMany, in radians plus
-// the scene's sizes. Milliseconds for 2^20 rays with one lane and with four: one instance, random 1.06, 1.19,
-// camera of 70 degrees 0.26, 0.39; 10 instances, random 4.0, 1.39, camera 0.44, 0.58; 100, camera 1.95, 1.49,
-// camera of 23 degrees 1.32, 1.79. 131,072 rays: 4 instances, camera 0.25, 0.21; 1 instance 0.19, 0.19.
+// coherent: 64 consecutive ones within kCoherentFew (up to kSceneFew instances) or kCoherentMany, or from within the
+// scene, where they meet fewer instances, kCoherentWithin, in radians plus the scene's sizes.
+// Milliseconds for 2^20 rays with one lane and with four: one instance, random 1.06, 1.19, camera of
+// 70 degrees 0.26, 0.39; 10 instances, random 4.0, 1.39, camera 0.44, 0.58; 100, camera 1.95, 1.49, within the
+// scene 1.12, 1.93, of 23 degrees 1.32, 1.79; 500, within the scene 2.5, 2.5. 131,072 rays: 4 instances, camera
+// 0.25, 0.21; 1 instance 0.19, 0.19.
 constexpr uint64_t kSceneOneLaneMin = 1u << 17;
 constexpr uint64_t kSceneSampleMin = 1u << 18;
-constexpr uint32_t kSceneFew = 32, kSceneSampled = 128;
-constexpr float kCoherentFew = 0.16f, kCoherentMany = 0.03f;
+constexpr uint32_t kSceneFew = 32, kSceneSampled = 256;
+constexpr float kCoherentFew = 0.16f, kCoherentMany = 0.03f, kCoherentWithin = 0.11f;
 
 struct mbvh_scene {
   uint32_t magic = 0x4E454353u;  // "SCEN"
   uint32_t n_listed = 0;           // visible instances
-  float per_size = 0.0f;           // 1 / the diagonal of their boxes
+  f3 box_lo{}, box_hi{};           // the box of their boxes
+  float per_size = 0.0f;           // 1 / its diagonal
   mbvh_ctx* ctx = nullptr;
   uint32_t n_meshes = 0;
   uint32_t n_instances = 0;
@@ -3286,6 +3289,8 @@ extern "C" int mbvh_scene_create(mbvh_ctx* ctx, const mbvh_mesh* const* meshes, 
   sc->similar = similar;
   sc->tlas_bound = tlas_bound;
   sc->n_listed = n_listed;
+  sc->box_lo = {box_lo[0], box_lo[1], box_lo[2]};
+  sc->box_hi = {box_hi[0], box_hi[1], box_hi[2]};
   sc->per_size = size > 0.0 ? static_cast<float>(1.0 / size) : 0.0f;
   sc->max_stack_points = max_stack_points;
   sc->max_stack_points4 = max_stack_points4;
@@ -3682,6 +3687,9 @@ int enqueue_scene(mbvh_ctx* ctx, const mbvh_scene* sc, const float* o, const flo
     if (a.n >= kSceneSampleMin && sc->n_listed <= kSceneSampled) {
       a.one_lane = static_cast<uint32_t*>(ctx->queue.ptr) + 50;
       a.coherent = sc->n_listed <= kSceneFew ? kCoherentFew : kCoherentMany;
+      a.coherent_within = sc->n_listed <= kSceneFew ? kCoherentFew : kCoherentWithin;
+      a.box_lo = sc->box_lo;
+      a.box_hi = sc->box_hi;
       a.per_size = sc->per_size;
     } else {
       a.one_lane = nullptr;

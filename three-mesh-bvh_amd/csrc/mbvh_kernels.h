@@ -301,9 +301,11 @@ struct SceneArgs {
   uint32_t* contender_pool_count;
   uint32_t contender_pool_cap;
   // raycast, four lanes: set, the launch first decides by the rays' coherence whether the one-lane kernel takes
-  // them all (*one_lane; a.n >= 4096): the spread up to which 64 rays are coherent, 1 / the scene's size
+  // them all (*one_lane; a.n >= 4096): the spread up to which 64 rays are coherent, from outside the box of the
+  // instances' boxes and from within it, that box, 1 / its diagonal
   uint32_t* one_lane;
-  float coherent;
+  float coherent, coherent_within;
+  f3 box_lo, box_hi;
   float per_size;
   const float* world;              // 16 floats per instance (local -> world, column-major)
   const float* inverse;            // 16 floats per instance (world -> local)

@@ -4835,8 +4835,8 @@ hipError_t launch_batch_raycast_first(const BatchArgs& a, uint32_t stack_lds, ui
 }
 
 // Clears the counters of a four-lane raycast and, where A.one_lane is set, decides whether one lane per ray takes
-// the call: where most of the samples, 64 consecutive rays each, stay within A.coherent (their directions'
-// spread and their origins' over the scene's size, added). Such rays share nodes within a wave of 64, which four
+// the call: where most of the samples, 64 consecutive rays each, stay within A.coherent or, from within the scene,
+// A.coherent_within (their directions' spread and their origins' over the scene's size, added). Such rays share nodes within a wave of 64, which four
 // lanes per ray make four times the steps of.
 __global__ __launch_bounds__(1024) void k_scene_reset(SceneArgs A) {
   if (threadIdx.x < kWalkQueues) A.queue[32 * threadIdx.x] = 0u;
@@ -4854,9 +4854,11 @@ __global__ __launch_bounds__(1024) void k_scene_reset(SceneArgs A) {
     const float per = __builtin_amdgcn_rsqf(dot(d, d));
     const f3 n = mk(d.x * per, d.y * per, d.z * per);
     const f3 dn = sub(n, mk(__shfl(n.x, 0, 64), __shfl(n.y, 0, 64), __shfl(n.z, 0, 64)));
-    const f3 dp = sub(o, mk(__shfl(o.x, 0, 64), __shfl(o.y, 0, 64), __shfl(o.z, 0, 64)));
+    const f3 o0 = mk(__shfl(o.x, 0, 64), __shfl(o.y, 0, 64), __shfl(o.z, 0, 64)), dp = sub(o, o0);
+    const bool within = o0.x >= A.box_lo.x && o0.x <= A.box_hi.x && o0.y >= A.box_lo.y && o0.y <= A.box_hi.y &&
+                        o0.z >= A.box_lo.z && o0.z <= A.box_hi.z;
     const float spread = __builtin_amdgcn_sqrtf(dot(dn, dn)) + __builtin_amdgcn_sqrtf(dot(dp, dp)) * A.per_size;
-    if (__ballot(spread <= A.coherent) == ~0ull && lane == 0) atomicAdd(&close, 1u);  // NaN: not close
+    if (__ballot(spread <= (within ? A.coherent_within : A.coherent)) == ~0ull && lane == 0) atomicAdd(&close, 1u);  // NaN: not close
   }
   __syncthreads();
   if (threadIdx.x == 0) *A.one_lane = 2 * close > kSamples ? 1u : 0u;
